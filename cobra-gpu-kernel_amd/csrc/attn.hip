@@ -45,10 +45,11 @@
 //   * the running sum adds the fp16 probabilities the P.V product consumes
 //     (v_dot2_f32_f16 against ones, fp32 accumulation), and the max/sum
 //     exchange with lane ^ 32 uses v_permlane32_swap;
-//   * key masks: the block's validity word is a scalar load (it waits in
-//     lgkmcnt, never behind the K/V transfers in vmcnt); a block without a
-//     valid key is skipped by the whole workgroup, a fully valid one costs a
-//     compare, and only partly valid blocks mask per key.
+//   * key masks: the block's validity words are scalar loads (they wait in
+//     lgkmcnt, never behind the K/V transfers in vmcnt).
+//
+// Two kernels share this layout: attn_fwd_kernel for non-causal calls and
+// attn_causal_kernel, where every wave's keys end elsewhere.
 // q, k, v and ctx are fp16 or bf16 (a template type): the bf16 form uses
 // v_mfma_f32_32x32x16_bf16 and v_dot2_f32_bf16 and rounds the probabilities to
 // bf16, everything else is the same code.
@@ -62,6 +63,17 @@ namespace {
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
+// 16 bytes at an LDS byte address.
+template <typename V>
+__device__ __forceinline__ V lds_read16(uint32_t addr) {
+  return *(__attribute__((address_space(3))) const V*)addr;
+}
+// The transposing 8-byte read at an LDS byte address.
+template <typename T>
+__device__ __forceinline__ typename Op16<T>::V4 lds_read_tr16(uint32_t addr) {
+  const s16x4 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)addr);
+  return __builtin_bit_cast(typename Op16<T>::V4, r);
+}
 template <typename T>
 __device__ __forceinline__ typename Op16<T>::V4 lds_read_tr16(const T* p) {
   const s16x4 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
@@ -87,8 +99,8 @@ __device__ __forceinline__ int swz(int row) {
   }
 }
 
-constexpr float kLazyRescale = 8.0f;  // log2 units
-constexpr float kAcceptSum = 65536.0f;  // a lane's tile sum accepted without a block max
+constexpr float kLazyRescale = 8.0f;    // log2 units
+constexpr float kAcceptSum = 65536.0f;  // a lane's tile sum accepted without a tile maximum
 
 __device__ __forceinline__ f32x16 splat16(float v) {
   f32x16 r;
@@ -99,7 +111,7 @@ __device__ __forceinline__ f32x16 splat16(float v) {
 
 }  // namespace
 
-template <int HD, int NW, int BN, int ST, bool CAUSAL, bool MASKED, typename TQ>
+template <int HD, int NW, int BN, int ST, bool MASKED, typename TQ>
 __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict__ qkv, TQ* __restrict__ ctx,
                                                            int S, int H, int hd, float c2, int nqb,
                                                            const uint64_t* __restrict__ key_bits, int nwords) {
@@ -149,7 +161,6 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, li = lane & 31;
   const int q0w = qb * BM + w * 32;  // this wave's first query
-  const int qi = q0w + li;           // this lane's query
 
   // Row-major [rows][HD] tiles in LDS, chunk c of row r at c ^ swz(r), filled by
   // coalesced LDS-DMA: 1 KB span `sp` of a tile holds rows sp*1024/(2HD) ..; each lane
@@ -217,8 +228,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
   const int vr = 4 * g + ((lane & 15) >> 2);
   const int vc = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
 
-  const int kend = CAUSAL ? min(S, (qb + 1) * BM) : S;
-  const int nblk = (kend + BN - 1) / BN;
+  const int nblk = (S + BN - 1) / BN;
   const int pre = min(ST - 1, nblk);  // key blocks in flight before the loop
   if constexpr (QSEP) {
 #pragma unroll
@@ -296,7 +306,8 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
     }
     lds_barrier();  // block n visible to all waves; every wave is done with block n-1
     if (n + ST - 1 < nblk) issue((n + ST - 1) % ST, (n + ST - 1) * BN);
-    bool kpart = false;  // some key of the block is padded
+    if (q0w >= S) continue;  // a wave past S only takes part in the transfers and barriers
+    bool kpart = false;      // some key of the block is padded
     if constexpr (MASKED) {
       constexpr uint64_t kFull = BN == 32 ? 0xffffffffull : ~0ull;
       uint64_t any = 0, all = kFull;
@@ -312,9 +323,8 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
     const TQ* Vc = reinterpret_cast<const TQ*>(smem + (n % ST) * SB + TB);
     // s = scores in the exp2 domain minus the running max: the accumulator
     // starts at -m_run (every register of a lane belongs to the lane's query).
-    // Masks only where a block reaches past S, causally past this wave's first
-    // query, or holds a padded key.
-    const bool need_mask = kb + BN > S || (CAUSAL && kb + BN > q0w + 1) || kpart;
+    // Masks only where a block reaches past S or holds a padded key.
+    const bool need_mask = kb + BN > S || kpart;
     auto scores = [&](f32x16(&s)[BN / 32]) {
 #pragma unroll
       for (int t = 0; t < BN / 32; ++t) {
@@ -328,13 +338,17 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
           s[t] = mfma32x32x16(a, qf[kk], s[t]);
         }
       }
+      // The compiler sizes its wait between a product and a vector read of the result by
+      // one of the paths that reach the read; with a single tile per block the shorter
+      // path is this branch alone, so wait here.
+      if constexpr (BN == 32) asm volatile("s_nop 7\n\ts_nop 3" : "+v"(s[0]));
       if (need_mask) {
         // Register r of tile t holds key kb + 4g + kc with kc = 32t + 8(r/4) + r%4,
-        // a constant: the key is past S or causally after the query iff kc > lim.
+        // a constant: the key is past S iff kc > lim.
         // A tile whose keys are all live for every lane of the wave is skipped
         // (a uniform branch per tile, which also keeps the predicates of one tile
         // at a time in scalar registers).
-        const int lim = CAUSAL ? min(S - 1, qi) - kb - 4 * g : S - 1 - kb - 4 * g;
+        const int lim = S - 1 - kb - 4 * g;
         uint64_t lw[KW];  // this lane's view: bit c = key kb + 32*(word half) + 4g + c
 #pragma unroll
         for (int k = 0; k < KW; ++k) lw[k] = MASKED ? kw[k] >> (4 * g) : 0;
@@ -460,6 +474,382 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
           const V8 a = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
           o[j] = mfma32x32x16(a, pf[kh], o[j]);
         }
+      }
+    }
+  }
+
+  // Output through LDS: O^T quads into [BM][HD] rows, then whole 16-byte chunks per
+  // lane, so the stores to ctx are row-contiguous.
+  const float l_tot = sum_xor32(l_run);
+  const float inv = MASKED ? (l_tot > 0.f ? 1.0f / l_tot : 0.f) : 1.0f / l_tot;
+  lds_barrier();  // every wave is done with the last stage
+#pragma unroll
+  for (int j = 0; j < ND; ++j)
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      const int d = j * 32 + 8 * q4 + 4 * g;
+      if (HD >= 32 || d < HD) {
+        const int row = w * 32 + li;
+        V4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = (TQ)(o[j][q4 * 4 + e] * inv);
+        *reinterpret_cast<V4*>(smem + row * 2 * HD + 16 * ((d >> 3) ^ swz<HD>(row)) + 8 * g) = v;
+      }
+    }
+  lds_barrier();
+  for (int idx = tid; idx < BM * CPR; idx += NT) {
+    const int row = idx / CPR, c = idx % CPR;
+    const int q = qb * BM + row, d0 = 8 * c;
+    if (q < S && d0 < hd)
+      *reinterpret_cast<V8*>(ctx + (b * S + q) * (int64_t)D + h * hd + d0) =
+          *reinterpret_cast<const V8*>(smem + row * 2 * HD + 16 * (c ^ swz<HD>(row)));
+  }
+}
+
+// The causal form, with or without key masks.  What it does otherwise than the kernel above:
+//   * keys come in pairs of 32-key tiles.  A pair whose keys are all live for every query
+//     of the wave takes the short path: scores, exponentials, products.  The references
+//     start at 0 rather than at a first block's maximum, so a wave's first pair takes it
+//     too when its sums lie in fp16's range.  Any other pair goes tile by tile through one
+//     straight line that masks, takes the tile's maximum and rescales; tiles without a live
+//     key are left out, by each wave for itself.
+//   * query blocks with the most keys are dispatched first (see below).
+//   * the reference is kept as the score products' C operand (16 registers) and LDS
+//     addresses stay in registers; with the masking out of the short path the kernel needs
+//     87-124 registers at head_dim <= 64 where one body with masks needed 124-158, so two
+//     workgroups of eight waves share a CU.
+// Measured in one process against that one-body form (us): causal B64 S1024 H4 hd32
+// 60 -> 49, B8 S2048 H16 hd64 140 -> 105, B8 S2048 H8 hd128 141 -> 99, B37 S333 H8 hd64
+// 34 -> 29.  Non-causal calls are no faster in this form (hd32 62 -> 63, hd64 1258 -> 1293 at
+// S16384, hd256 56 -> 69) and keep the kernel above.  Bound by the overlap of the matrix and
+// vector pipes: at hd64 each is busy half of the time, and fewer vector instructions, LDS
+// waits or barriers did not move it.
+template <int HD, int NW, int BN, int ST, bool MASKED, typename TQ>
+__global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_causal_kernel(const TQ* __restrict__ qkv, TQ* __restrict__ ctx,
+                                                           int S, int H, int hd, float c2, int nqb,
+                                                           const uint64_t* __restrict__ key_bits, int nwords) {
+  using V8 = typename Op16<TQ>::V8;
+  using V4 = typename Op16<TQ>::V4;
+  using V2 = typename Op16<TQ>::V2;
+  constexpr int BM = 32 * NW;          // queries per workgroup
+  constexpr int KS = HD / 16;          // k-steps of the QK^T product
+  constexpr int ND = (HD + 31) / 32;   // 32-row blocks of d in O^T
+  constexpr int NT = NW * 64;
+  constexpr int CPR = HD / 8;          // 16-byte chunks per row
+  constexpr int TB = BN * HD * 2;      // bytes of one K (or V) tile
+  constexpr int SB = 2 * TB;           // bytes of one stage: K tile, then V tile
+  constexpr int NI = SB / 1024;        // 1 KB DMA spans per stage
+  constexpr int LPT = NI / NW;         // spans per wave per stage
+  constexpr int QPT = BM * HD * 2 / 1024 / NW;  // Q-tile spans per wave
+  static_assert(HD % 16 == 0 && BN % 32 == 0, "tile geometry");
+  static_assert(BN == 32 || BN % 64 == 0, "key-mask words");
+  constexpr int KW = BN > 64 ? BN / 64 : 1;  // validity words per key block
+  constexpr int NTL = BN / 32;         // 32-key tiles per block
+  constexpr int PT = NTL < 2 ? 1 : 2;  // tiles whose scores are in flight together
+  static_assert(NI % (2 * NW) == 0, "every wave DMAs whole spans of each tile");
+  // Short-sequence launches (<= 4 waves) give the Q tile its own LDS region, so its
+  // DMA overlaps the first K/V stages instead of preceding them; 8-wave launches
+  // (long sequences) stage it through the K/V stages to keep LDS small.
+  constexpr bool QSEP = NW <= 4;
+  constexpr int QB = BM * HD * 2;
+  constexpr int LDSB = ST * SB + (QSEP ? QB : 0);
+  static_assert(BM * HD * 2 <= ST * SB, "the output tile passes through the K/V stages");
+  static_assert(ST >= 2 && (ST - 1) * LPT < 64, "vmcnt range");
+  static_assert(LDSB <= 163840, "LDS budget");
+
+  __shared__ __attribute__((aligned(1024))) char smem[LDSB];
+  char* const qtile = smem + (QSEP ? ST * SB : 0);
+
+  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  // Query block qb visits qb + 1 blocks' worth of keys: of every eight (sequence, head)
+  // pairs the long ones are dispatched first, so that the short ones fill the end.  Eight,
+  // because a group's workgroups share the K / V of its pairs in their XCD's L2.
+  const int grp = id / (8 * nqb), in_grp = id - grp * 8 * nqb;
+  const int pairs = min(8, (int)(gridDim.x / nqb) - 8 * grp);
+  const int qb = nqb - 1 - in_grp / pairs;
+  const int bh = 8 * grp + in_grp % pairs;
+  const int h = bh % H;
+  const int64_t b = bh / H;
+  const int D = H * hd;
+  const int64_t ld = 3 * (int64_t)D;
+  const TQ* qbase = qkv + b * S * ld + h * hd;
+  const TQ* kbase = qbase + D;
+  const TQ* vbase = qbase + 2 * D;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 5, li = lane & 31;
+  const int q0w = qb * BM + w * 32;  // this wave's first query
+  const int qi = q0w + li;           // this lane's query
+
+  // Row-major [rows][HD] tiles in LDS, chunk c of row r at c ^ swz(r), filled by
+  // coalesced LDS-DMA: 1 KB span `sp` of a tile holds rows sp * RPS ..; each lane fetches
+  // the global chunk that belongs in its slot.  Rows past S fetch row S-1 and chunks past
+  // hd fetch chunk 0 (finite values; masked, zero-weighted or not stored).
+  // A span is one uniform base (its first row) plus the lane's byte offset.
+  constexpr int RPS = 512 / HD;  // rows per span
+  const uint32_t ldb = (uint32_t)ld * 2;
+  const uint32_t lds0 = lds_addr(smem);
+  auto span_row = [&](int sp, int last) { return min(sp * RPS, last); };
+  auto span_off = [&](int sp, int last) {
+    const int row = sp * RPS + 16 * lane / (2 * HD), pos = (16 * lane % (2 * HD)) / 16;
+    const int d0 = 8 * (pos ^ swz<HD>(row));
+    return (uint32_t)(min(row, last) - span_row(sp, last)) * ldb + (d0 < hd ? 2 * d0 : 0);
+  };
+
+  // Q^T fragments: B operand of S^T = K . Q^T (k = d), staged through LDS and
+  // pre-scaled by scale * log2(e) so that the products come out in the exp2 domain.
+#pragma unroll
+  for (int i = 0; i < QPT; ++i) {
+    const int sp = w + NW * i, last = S - 1 - qb * BM;
+    dma16_untracked(qbase + (int64_t)(qb * BM + span_row(sp, last)) * ld, span_off(sp, last),
+                    lds_addr(qtile) + sp * 1024);
+  }
+
+  // K/V stages: ST tiles deep, one barrier per key block.  Wave w moves spans w, w + NW, ..
+  // of the K tile and of the V tile.
+  constexpr int KPT = LPT / 2;  // spans per wave per tile
+  uint32_t koff[KPT];
+#pragma unroll
+  for (int i = 0; i < KPT; ++i) koff[i] = span_off(w + NW * i, BN - 1);
+  auto issue = [&](int stage, int kb) {
+    const uint32_t dst = lds0 + stage * SB + w * 1024;
+    const bool whole = kb + BN <= S;
+    const int last = whole ? BN - 1 : S - 1 - kb;
+#pragma unroll
+    for (int i = 0; i < KPT; ++i) {
+      const int sp = w + NW * i;
+      const int64_t row = (int64_t)(kb + span_row(sp, last)) * ld;
+      uint32_t off = koff[i];
+      if (!whole) off = span_off(sp, last);
+      dma16_untracked(kbase + row, off, dst + NW * i * 1024);
+      dma16_untracked(vbase + row, off, dst + TB + NW * i * 1024);
+    }
+  };
+
+  f32x16 o[ND];
+#pragma unroll
+  for (int j = 0; j < ND; ++j) o[j] = zero16();
+  // The softmax reference of this lane's query, negated: what every score tile starts
+  // from.  KEEP: repeated in 16 registers as the products' C operand, opaque to the
+  // compiler, which would otherwise rebuild the copies for every tile.
+  constexpr bool KEEP = PT <= 2 && HD <= 128;
+  f32x16 negm = splat16(0.f);
+  if constexpr (KEEP) asm volatile("" : "+v"(negm));
+  float l_run = 0.f;     // this lane's share of the running sum
+  bool settled = false;  // every query of the wave has a reference (wave-uniform)
+  const uint64_t* krow = MASKED ? key_bits + b * nwords : nullptr;
+  const V2 ones = {(TQ)1.0f, (TQ)1.0f};
+
+  // LDS byte offsets of this lane's operand reads in stage 0: the K fragments of the first
+  // tile's k-steps, and per d-tile the two halves of a V^T fragment of its first 16 keys
+  // (row within a 16-key step vr, column within a 32-wide d tile vc; see the header).
+  // Opaque, so that they stay in registers: the compiler would form them again per tile.
+  const int vr = 4 * g + ((lane & 15) >> 2);
+  const int vc = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  uint32_t ka[KS], va[ND], vb[ND];
+#pragma unroll
+  for (int kk = 0; kk < KS; ++kk) {
+    ka[kk] = lds0 + li * 2 * HD + 16 * ((2 * kk + g) ^ swz<HD>(li));
+    asm volatile("" : "+v"(ka[kk]));
+  }
+#pragma unroll
+  for (int j = 0; j < ND; ++j) {
+    const int c = j * 32 + (HD >= 32 ? vc : vc & 15);
+    va[j] = lds0 + TB + vr * 2 * HD + 16 * ((c >> 3) ^ swz<HD>(vr)) + 2 * (c & 7);
+    vb[j] = lds0 + TB + (vr + 8) * 2 * HD + 16 * ((c >> 3) ^ swz<HD>(vr + 8)) + 2 * (c & 7);
+    asm volatile("" : "+v"(va[j]), "+v"(vb[j]));
+  }
+
+  const int kend = min(S, (qb + 1) * BM);
+  const int nblk = (kend + BN - 1) / BN;
+  const int pre = min(ST - 1, nblk);  // key blocks in flight before the loop
+  // Wait until at most n blocks' transfers are in flight.
+  auto wait_blocks = [&](int n) {
+    if (ST >= 4 && n >= 3) {
+      wait_vmcnt<(ST >= 4 ? 3 : 0) * LPT>();
+    } else if (ST >= 3 && n >= 2) {
+      wait_vmcnt<(ST >= 3 ? 2 : 0) * LPT>();
+    } else if (n >= 1) {
+      wait_vmcnt<LPT>();
+    } else {
+      wait_vmcnt<0>();
+    }
+  };
+  if constexpr (QSEP) {
+#pragma unroll
+    for (int s = 0; s < ST - 1; ++s)
+      if (s < nblk) issue(s, s * BN);
+    wait_blocks(pre);  // the Q tile is the oldest transfer: wait for it alone
+  } else {
+    wait_vmcnt<0>();
+  }
+  stage_barrier();
+  V8 qf[KS];
+#pragma unroll
+  for (int kk = 0; kk < KS; ++kk) {
+    const int row = w * 32 + li, d0 = kk * 16 + g * 8;
+    const V8 q = *reinterpret_cast<const V8*>(qtile + row * 2 * HD + 16 * ((2 * kk + g) ^ swz<HD>(row)));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) qf[kk][e] = d0 < hd ? (TQ)((float)q[e] * c2) : (TQ)0.0f;
+  }
+  if constexpr (!QSEP) {
+    lds_barrier();  // every wave has its Q fragments before the stages are refilled
+#pragma unroll
+    for (int s = 0; s < ST - 1; ++s)
+      if (s < nblk) issue(s, s * BN);
+  }
+  for (int n = 0; n < nblk; ++n) {
+    const int kb = n * BN;
+    // Validity words of the block's keys, one per 64; the scalar loads complete under the
+    // barrier's lgkmcnt wait below.
+    uint64_t kw[KW];
+    if constexpr (MASKED) {
+#pragma unroll
+      for (int k = 0; k < KW; ++k) {
+        const int wi = (kb >> 6) + k;
+        kw[k] = krow[min(wi, nwords - 1)];
+        if (wi >= nwords) kw[k] = 0;
+      }
+      if constexpr (BN == 32) kw[0] = (kw[0] >> (kb & 32)) | 0xffffffff00000000ull;
+    }
+    // Blocks n+1 .. n+ST-2 may still be in flight; block n must have landed.
+    wait_blocks(min(ST - 2, nblk - 1 - n));
+    lds_barrier();  // block n visible to all waves; every wave is done with block n-1
+    if (n + ST - 1 < nblk) issue((n + ST - 1) % ST, (n + ST - 1) * BN);
+    if (q0w >= S || kb > q0w + 31) continue;  // nothing of this block for this wave
+    const uint32_t base = (n % ST) * SB;
+    // Scores of a key tile in the exp2 domain, relative to the queries' references.
+    auto scores = [&](f32x16& s, uint32_t at) {
+      s = KEEP ? negm : splat16(negm[0]);
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) s = mfma32x32x16(lds_read16<V8>(ka[kk] + at), qf[kk], s);
+    };
+    // p = exp2(s) rounded to the operand type, in the P.V B-operand layout (two 16-key
+    // steps); returns this lane's share of the tile's row sum over those rounded values
+    // (the ones the P.V product uses), accumulated in fp32.
+    auto probs = [&](const f32x16& s, V8(&pf)[2]) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) pf[r >> 3][r & 7] = (TQ)__builtin_amdgcn_exp2f(s[r]);
+      float lt = 0.f;
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const V2 pr = {pf[k][2 * e], pf[k][2 * e + 1]};
+          lt = dot2(pr, ones, lt);
+        }
+      return lt;
+    };
+    // No tile maximum: the probabilities are formed against the query's reference (0 to
+    // begin with) and accepted when every lane's tile sum is at most 2^16, so that no
+    // probability exceeds 2^16 (fp16 holds each one; an fp16 overflow reads as an infinite
+    // sum), and, until every query of the wave has a sum, when each has one of at least
+    // 1/2, so that none is lost at fp16's small end.
+    auto accepted = [&](float lt, bool first) {
+      bool refused = __builtin_amdgcn_ballot_w64(!(lt <= kAcceptSum)) != 0;
+      if (first && !settled)
+        refused = refused || __builtin_amdgcn_ballot_w64(!(sum_xor32(l_run + lt) >= 0.5f)) != 0;
+      return !refused;
+    };
+    auto pv = [&](const V8(&pf)[2], uint32_t at) {
+#pragma unroll
+      for (int kh = 0; kh < 2; ++kh) {
+#pragma unroll
+        for (int j = 0; j < ND; ++j) {
+          const V4 lo = lds_read_tr16<TQ>(va[j] + at + kh * 32 * HD);
+          const V4 hi = lds_read_tr16<TQ>(vb[j] + at + kh * 32 * HD);
+          const V8 a = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+          o[j] = mfma32x32x16(a, pf[kh], o[j]);
+        }
+      }
+    };
+#pragma unroll 1
+    for (int tp = 0; tp < NTL; tp += PT) {
+      const int kp = kb + 32 * tp;  // first key of these tiles
+      if (kp >= S || kp > q0w + 31) break;
+      uint64_t word = ~0ull;  // validity of keys kp .. kp + 63
+      if constexpr (MASKED) {
+        word = kw[0];
+#pragma unroll
+        for (int k = 1; k < KW; ++k) word = tp == 2 * k ? kw[k] : word;
+        if (word == 0) continue;
+      }
+      const uint32_t at = base + tp * 64 * HD;
+      int done = 0;
+      // Every key of the tiles is live for every query of the wave.
+      if (kp + 32 * PT <= S && kp + 32 * PT <= q0w + 1 && (!MASKED || word == ~0ull)) {
+        // All scores first, and a tile's P.V products overlap the next one's exponentials.
+        f32x16 s[PT];
+#pragma unroll
+        for (int u = 0; u < PT; ++u) scores(s[u], at + u * 64 * HD);
+#pragma unroll
+        for (int u = 0; u < PT; ++u) {
+          if (done == u) {
+            V8 pf[2];
+            const float lt = probs(s[u], pf);
+            if (accepted(lt, u == 0)) {
+              l_run += lt;
+              settled = true;
+              pv(pf, at + u * 64 * HD);
+              done = u + 1;
+            }
+          }
+        }
+      }
+      // The other tiles, one at a time with their maximum: those refused, and those of
+      // blocks that reach past S, past the wave's first query (causal) or hold padded
+      // keys.  Register r of tile t holds key k0 + 4g + kc, kc = 8(r/4) + r%4: past S or
+      // causally after the query iff kc > lim.  One straight line, the rescale included
+      // (by 1 where no reference moves): branches here made the compiler keep second
+      // copies of O and the references on the path above.
+#pragma unroll 1
+      for (int t = done; t < PT; ++t) {
+        const int k0 = kp + 32 * t;
+        if (k0 >= S || k0 > q0w + 31) break;
+        uint32_t tw = ~0u;  // validity of keys k0 .. k0 + 31
+        if constexpr (MASKED) {
+          tw = (uint32_t)(word >> (32 * t));
+          if (tw == 0) continue;
+          tw >>= 4 * g;
+        }
+        f32x16 s;
+        scores(s, at + t * 64 * HD);
+        const int lim = min(S - 1, qi) - k0 - 4 * g;
+        float mx = kNegInf;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int kc = 8 * (r >> 2) + (r & 3);
+          bool dead = kc > lim;
+          if constexpr (MASKED) dead = dead || !((tw >> kc) & 1);
+          if (dead) s[r] = kNegInf;
+          mx = fmaxf(mx, s[r]);
+        }
+        mx = max_xor32(mx);  // relative to the reference; both lanes of a query agree
+        // A query without a sum yet takes the tile's maximum as its reference; one with a
+        // sum moves only when the tile lies more than kLazyRescale above it.
+        const bool fresh = !(sum_xor32(l_run) > 0.f);
+        const float inc = fresh ? (mx != kNegInf ? mx : 0.f) : (mx > kLazyRescale ? mx : 0.f);
+        const float alpha = fresh ? 1.f : __builtin_amdgcn_exp2f(-inc);
+        l_run *= alpha;
+#pragma unroll
+        for (int j = 0; j < ND; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[j][r] *= alpha;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] -= inc;
+        if constexpr (KEEP) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) negm[r] -= inc;
+          asm volatile("" : "+v"(negm));
+        } else {
+          negm = splat16(negm[0] - inc);
+        }
+        V8 pf[2];
+        l_run += probs(s, pf);
+        settled = !__builtin_amdgcn_ballot_w64(!(sum_xor32(l_run) > 0.f));
+        pv(pf, at + t * 64 * HD);
       }
     }
   }
@@ -674,44 +1064,48 @@ static hipError_t launch_attn_short(const AttnArgs& a, float c2) {
   return hipGetLastError();
 }
 
-template <int HD, int NW, int BN, int ST, bool CAUSAL, typename TQ>
+template <int HD, int NW, int BN, int ST, bool CAUSAL, bool MASKED, typename TQ>
 static hipError_t launch_attn(const AttnArgs& a, float c2) {
-  constexpr int BM = 32 * NW;
-  const int nqb = (a.seq_len + BM - 1) / BM;
+  const int nqb = (a.seq_len + 32 * NW - 1) / (32 * NW);
   const int64_t grid = (int64_t)nqb * a.heads * a.batch;
   if (grid > 0x7fffffff) return hipErrorInvalidValue;
-  const int nwords = (int)mask_words(a.seq_len);
-  if (a.key_bits)
-    hipLaunchKernelGGL((attn_fwd_kernel<HD, NW, BN, ST, CAUSAL, true, TQ>), dim3((unsigned)grid), dim3(NW * 64), 0,
-                       a.stream, static_cast<const TQ*>(a.qkv), static_cast<TQ*>(a.ctx), a.seq_len, a.heads,
-                       a.head_dim, c2, nqb, a.key_bits, nwords);
-  else
-    hipLaunchKernelGGL((attn_fwd_kernel<HD, NW, BN, ST, CAUSAL, false, TQ>), dim3((unsigned)grid), dim3(NW * 64), 0,
-                       a.stream, static_cast<const TQ*>(a.qkv), static_cast<TQ*>(a.ctx), a.seq_len, a.heads,
-                       a.head_dim, c2, nqb, nullptr, nwords);
+  auto* const kernel = [] {
+    if constexpr (CAUSAL) return attn_causal_kernel<HD, NW, BN, ST, MASKED, TQ>;
+    else return attn_fwd_kernel<HD, NW, BN, ST, MASKED, TQ>;
+  }();
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(NW * 64), 0, a.stream, static_cast<const TQ*>(a.qkv),
+                     static_cast<TQ*>(a.ctx), a.seq_len, a.heads, a.head_dim, c2, nqb, a.key_bits,
+                     (int)mask_words(a.seq_len));
   return hipGetLastError();
+}
+
+// Waves per workgroup follow the sequence length: every K/V tile a workgroup stages is
+// shared by all of its waves, so long sequences take 8 (256 queries), short ones fewer so
+// that no wave idles past S.  Wide heads keep 4: the O accumulator already fills the
+// register file.  Key blocks of BN keys, ST stages deep: 8-wave launches need at least one
+// 1 KB DMA span per wave per stage (the causal kernel: of the K and of the V tile), and
+// narrow heads take 128-key blocks (half the barriers per key; +7-10 % at head_dim 32,
+// measured).
+template <int HD, bool CAUSAL, bool MASKED, typename TQ>
+static hipError_t dispatch_waves(const AttnArgs& a, float c2) {
+  constexpr int BN = HD >= 256 ? 32 : 64;
+  constexpr int BN4 = CAUSAL && HD <= 16 ? 128 : BN;
+  constexpr int BN8 = CAUSAL ? (HD <= 16 ? 256 : 128) : (HD <= 32 ? 128 : BN);
+  constexpr int ST = CAUSAL || HD >= 128 ? 3 : 4;
+  constexpr int ST8 = CAUSAL && HD != 32 ? 2 : HD >= 128 ? 3 : 4;
+  if constexpr (HD <= 64) {
+    if (a.seq_len <= 32) return launch_attn<HD, 1, BN, ST, CAUSAL, MASKED, TQ>(a, c2);
+    if (a.seq_len <= 64) return launch_attn<HD, 2, BN, ST, CAUSAL, MASKED, TQ>(a, c2);
+  }
+  if constexpr (HD <= 128) {
+    if (a.seq_len > 128) return launch_attn<HD, 8, BN8, ST8, CAUSAL, MASKED, TQ>(a, c2);
+  }
+  return launch_attn<HD, 4, BN4, ST, CAUSAL, MASKED, TQ>(a, c2);
 }
 
 template <int HD, bool CAUSAL, typename TQ>
 static hipError_t dispatch_waves(const AttnArgs& a, float c2) {
-  // Waves per workgroup follow the sequence length: every K/V tile a
-  // workgroup stages is shared by all of its waves, so long sequences take 8
-  // (256 queries), short ones fewer so that no wave idles past S.  Wide heads
-  // keep 4: the O accumulator already fills the register file.  Key blocks of
-  // BN keys (one 1 KB DMA span per wave at least), ST stages deep.
-  constexpr int BN = HD >= 256 ? 32 : 64;
-  // 8-wave launches: at least one 1 KB span per wave per stage, and for narrow heads
-  // 128-key blocks (half the barriers per key; +7-10 % at head_dim 32, measured)
-  constexpr int BN8 = HD <= 32 ? 128 : BN;
-  constexpr int ST = HD >= 128 ? 3 : 4;
-  if constexpr (HD <= 64) {
-    if (a.seq_len <= 32) return launch_attn<HD, 1, BN, ST, CAUSAL, TQ>(a, c2);
-    if (a.seq_len <= 64) return launch_attn<HD, 2, BN, ST, CAUSAL, TQ>(a, c2);
-  }
-  if constexpr (HD <= 128) {
-    if (a.seq_len > 128) return launch_attn<HD, 8, BN8, ST, CAUSAL, TQ>(a, c2);
-  }
-  return launch_attn<HD, 4, BN, ST, CAUSAL, TQ>(a, c2);
+  return a.key_bits ? dispatch_waves<HD, CAUSAL, true, TQ>(a, c2) : dispatch_waves<HD, CAUSAL, false, TQ>(a, c2);
 }
 
 template <bool CAUSAL, typename TQ>

@@ -17,6 +17,23 @@ __device__ __forceinline__ void dma16(const void* src, void* lds_base) {
   __builtin_amdgcn_global_load_lds(src, (lds_ptr)lds_base, 16, 0, 0);
 }
 
+// 16 bytes per lane from base + off (a wave-uniform base, a per-lane byte offset) to
+// lds + 16 * lane, issued where the compiler does not see an LDS write: it cannot tell one
+// pipeline stage from another, and puts a wait for every transfer in flight (vmcnt(0)) in
+// front of the transposing LDS reads that follow a dma16.  For kernels whose own wait_vmcnt
+// and barriers order every transfer against the reads of its stage.  No register is
+// written, so nothing has to outlive the transfer; the uniform base costs no vector
+// arithmetic per transfer.  M0 cannot be named as clobbered (a reserved register): a kernel
+// that uses this must not also use dma16, whose M0 the compiler sets and may keep.
+__device__ __forceinline__ void dma16_untracked(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds), "v"(off), "s"(base)
+               : "memory");
+}
+// LDS byte address of a shared-memory pointer.
+__device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(lds_ptr)p; }
+
 // s_waitcnt vmcnt(n), leaving the other counters unconstrained (gfx9 encoding).
 // The empty asm statement keeps the compiler from hoisting reads of the DMA'd
 // LDS above the wait.

@@ -1,0 +1,86 @@
+"""GPU checks of the causal and the key-masked attention where blocks and tiles end.
+
+Sequence lengths on both sides of a 32-key tile, a 64-key mask word, a 128-key block and a
+256-query workgroup; every head-dim class and some head dims below their class's width;
+token masks that end a sequence early, start it late, leave holes, or empty it; and logits
+moved far up and down, so that a wave's first tiles are refused and its references move
+(an added constant per query leaves the softmax itself unchanged).
+
+Reference: fp32 torch softmax attention on the same 16-bit values (TTB:98-113); gate of the
+other attention op tests (`allclose(atol=2e-3, rtol=1e-2)`, bf16 `atol=1.6e-2, rtol=2e-2`:
+the rounding of the probabilities and of the output, 2^-11 / 2^-8 of values of order 1).
+"""
+
+import pytest
+import torch
+
+from _gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+
+
+def _mask(kind, B, S, g):
+    j = torch.arange(S)[None, :]
+    if kind == "none":
+        return None
+    if kind == "tail":
+        return j < torch.randint(1, S + 1, (B, 1), generator=g)
+    if kind == "head":
+        return j >= torch.randint(0, S, (B, 1), generator=g)
+    m = torch.rand(B, S, generator=g) < 0.6
+    m[0] = False
+    return m
+
+
+def _reference(qkv, B, S, H, hd, causal, mask):
+    q, k, v = qkv.float().view(B, S, 3, H, hd).permute(2, 0, 3, 1, 4)
+    s = (q @ k.transpose(-2, -1).contiguous()) * hd ** -0.5
+    dead = torch.zeros(B, 1, S, S, dtype=torch.bool, device=qkv.device)
+    if mask is not None:
+        dead = dead | ~mask[:, None, None, :]
+    if causal:
+        dead = dead | torch.ones(S, S, dtype=torch.bool, device=qkv.device).triu(1)
+    p = torch.softmax(s.masked_fill(dead, float("-inf")), -1).nan_to_num(0.0)
+    return (p @ v).transpose(1, 2).reshape(B * S, H * hd)
+
+
+@pytest.mark.parametrize("hd", [8, 16, 32, 40, 64, 128, 200, 256])
+@pytest.mark.parametrize("causal,kind", [(True, "none"), (False, "tail"), (True, "tail"), (True, "head"),
+                                         (False, "holes"), (True, "holes")])
+@pytest.mark.parametrize("offset", [0.0, 40.0, -40.0])
+def test_attn_edges(hd, causal, kind, offset):
+    from cobra_amd import ops
+
+    B, H = 3, 2
+    for S in (1, 31, 33, 64, 65, 127, 129, 256, 257, 333):
+        g = torch.Generator().manual_seed(S * 7 + hd)
+        q, k, v = torch.randn(3, B, S, H, hd, generator=g)
+        if offset:
+            q[..., 0], k[..., 0] = hd ** 0.5, offset  # adds `offset` to every logit
+        qkv = torch.stack([q, k, v], 2).reshape(B * S, 3 * H * hd)
+        mask = _mask(kind, B, S, g)
+        for dt in (torch.float16, torch.bfloat16) if offset == 0.0 else (torch.float16,):
+            x = qkv.to(dt).to(DEV)
+            m = None if mask is None else mask.to(DEV)
+            got = ops.attn(x, B, S, H, hd, hd ** -0.5, causal=causal, key_mask=m).float()
+            want = _reference(x, B, S, H, hd, causal, m)
+            tol = dict(atol=2e-3, rtol=1e-2) if dt == torch.float16 else dict(atol=1.6e-2, rtol=2e-2)
+            err = (got - want).abs().max().item()
+            assert torch.allclose(got, want, **tol), (hd, S, causal, kind, offset, dt, err)
+    print(f"[attn-edges] hd{hd} causal={causal} mask={kind} offset={offset} ok", flush=True)
+
+
+@pytest.mark.parametrize("hd", [64, 256])
+def test_masked_attention_repeats_bit_for_bit(hd):
+    """Sharp logits and a mask ending inside a tile: references move at many places, and two
+    launches agree bit for bit (each output has one owner and a fixed order of sums)."""
+    from cobra_amd import ops
+
+    B, S, H = 4, 1001, 2
+    g = torch.Generator().manual_seed(hd)
+    x = (torch.randn(B * S, 3 * H * hd, generator=g) * 2.0).half().to(DEV)
+    mask = (torch.arange(S)[None, :] < torch.tensor([[1001], [870], [613], [40]])).to(DEV)
+    got = ops.attn(x, B, S, H, hd, hd ** -0.5, causal=False, key_mask=mask)
+    assert torch.equal(got, ops.attn(x, B, S, H, hd, hd ** -0.5, causal=False, key_mask=mask))
+    want = _reference(x, B, S, H, hd, False, mask)
+    assert torch.allclose(got.float(), want, atol=8e-3, rtol=1e-2)  # v is twice as large, p up to 1: 4x the rounding
