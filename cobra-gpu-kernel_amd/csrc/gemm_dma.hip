@@ -1,5 +1,5 @@
-// C[M,N] = A[M,K] . W[N,K]^T (+ bias[N]) (+ resid[M,N]) for the large
-// projections: fp16 or bf16 operands, fp32 accumulate, C in the operand type or fp32.
+// C[M,N] = A[M,K] . W[N,K]^T (+ bias[N]) (+ resid[M,N]) for N and K in groups of 8: fp16
+// or bf16 operands, fp32 accumulate, C in the operand type or fp32.
 //
 // Same contract as the register-staged GEMM (replaces the reference's
 // _gemm_kernel / _tl_linear, torch_transformer_benchmark.py:283-381): each
@@ -12,10 +12,12 @@
 //     16-byte chunks (chunk c of row r at c ^ ((r >> 1) & 7)); since the DMA
 //     destination of a lane is fixed (band base + 16 * lane), each lane instead
 //     fetches the global chunk that belongs in its slot;
-//   * ST stages of LDS, one barrier per k-tile: a wave waits for its own DMA
-//     of tile kt (vmcnt), the barrier makes every wave's DMA visible and
-//     retires the stage computed in the previous step, which then receives
-//     tile kt + ST - 1;
+//   * ST stages of LDS, one barrier per k-tile: it stands where a wave has read all its
+//     fragments of tile kt and its own DMA of tile kt + 1 has landed (vmcnt), makes every
+//     wave's DMA visible and retires tile kt's stage, which then receives tile kt + ST;
+//     the products of tile kt's last k-step and the first LDS reads of the next tile
+//     run past it.  The DMA is issued untracked (lds_dma.hpp): with transfers the compiler
+//     knows of in flight it made every wait on an LDS read a wait for all of them;
 //   * v_mfma_f32_32x32x16_f16 (_bf16) with the weight tile as the A operand, so the
 //     accumulator holds C^T: each lane owns one output row and 4 consecutive
 //     columns per register quad;
@@ -52,6 +54,9 @@ struct DmaTile {
   static_assert(BM % 16 == 0 && BN % 16 == 0, "swizzle period");
   static_assert(LDS <= 163840, "LDS budget");
 };
+
+// What a chunk past the end of K reads.
+__device__ const uint4 kZeroChunk[1] = {};
 
 __device__ __forceinline__ int chunk_swz(int row) { return (row >> 1) & 7; }
 
@@ -97,14 +102,21 @@ __device__ __forceinline__ void dma_mainloop(const TA* __restrict__ A, const TA*
       src_off[i] = (unsigned)(((int64_t)n * K + chunk * 8) * 2);
     }
   }
+  const uint32_t lds0 = lds_addr(smem);
   auto issue = [&](int stage, int k0) {
-    char* sbase = smem + stage * T::STAGE * 2;
+    const uint32_t dst = lds0 + stage * T::STAGE * 2 + wave * 1024;
+    if (k0 + BK <= K) {
 #pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const int band = wave + i * NW;
-      const char* src = (8 * band < BM ? reinterpret_cast<const char*>(Ablk) : reinterpret_cast<const char*>(Wblk)) +
-                        (int64_t)k0 * 2 + src_off[i];
-      dma16(src, sbase + band * 1024);
+      for (int i = 0; i < LPT; ++i)
+        dma16_untracked((8 * (wave + i * NW) < BM ? Ablk : Wblk) + k0, src_off[i], dst + i * NW * 1024);
+    } else {  // the last k-tile when K % 64 != 0: chunks past K (a multiple of 8) are zero
+#pragma unroll
+      for (int i = 0; i < LPT; ++i) {
+        const int row = 8 * (wave + i * NW) + (lane >> 3);
+        const char* src = reinterpret_cast<const char*>((8 * (wave + i * NW) < BM ? Ablk : Wblk) + k0) + src_off[i];
+        if (k0 + 8 * ((lane & 7) ^ chunk_swz(row)) >= K) src = reinterpret_cast<const char*>(kZeroChunk);
+        dma16_untracked(src, dst + i * NW * 1024);
+      }
     }
   };
 
@@ -119,43 +131,59 @@ __device__ __forceinline__ void dma_mainloop(const TA* __restrict__ A, const TA*
   const int arow = (wm * T::WTM + li) * BK;
   const int wrow = (BM + wn * T::WTN + li) * BK;
 
-  const int KT = K / BK;
+  const int KT = (K + BK - 1) / BK;
 #pragma unroll
-  for (int s = 0; s < ST - 1; ++s)
+  for (int s = 0; s < ST; ++s)
     if (s < KT) issue(s, s * BK);
 
-  for (int kt = 0; kt < KT; ++kt) {
-    if constexpr (ST >= 3) {
-      if (kt + 1 < KT) {
-        wait_vmcnt<(ST - 2) * LPT>();
-      } else {
-        wait_vmcnt<0>();
-      }
+  // Operand fragments double-buffered across the 16-deep k-steps, over the k-tile boundary
+  // too: step kk's products run while step kk + 1's LDS reads are in flight.  Before the
+  // last step's products of a tile its reads are all done, so there the barrier retires the
+  // stage: it is refilled at once with tile kt + ST, and the next tile's first reads are
+  // under way during those products.  (Left to itself the compiler gives both buffers the
+  // same registers and waits for every read in front of every group of products; the
+  // scheduling barriers keep the order as written.)
+  V8 af[2][T::TM], wf[2][T::TN];
+  auto frags = [&](const TA* sa, int kk, int b) {
+    const int co = ((2 * kk + g) ^ sw) * 8;
+#pragma unroll
+    for (int j = 0; j < T::TN; ++j) wf[b][j] = *reinterpret_cast<const V8*>(sa + wrow + j * 32 * BK + co);
+#pragma unroll
+    for (int i = 0; i < T::TM; ++i) af[b][i] = *reinterpret_cast<const V8*>(sa + arow + i * 32 * BK + co);
+  };
+  // Wait for the oldest tile in flight, of which there are n.
+  auto wait_oldest = [&](int n) {
+    if (ST >= 4 && n >= 4) {
+      wait_vmcnt<(ST >= 4 ? 3 : 0) * LPT>();
+    } else if (ST >= 3 && n >= 3) {
+      wait_vmcnt<(ST >= 3 ? 2 : 0) * LPT>();
+    } else if (n >= 2) {
+      wait_vmcnt<LPT>();
     } else {
       wait_vmcnt<0>();
     }
-    stage_barrier();
-    if (kt + ST - 1 < KT) issue((kt + ST - 1) % ST, (kt + ST - 1) * BK);
-
-    // Operand fragments double-buffered across the four 16-deep k-steps: the
-    // LDS reads of step kk + 1 are in flight during the MFMAs of step kk.
+  };
+  wait_oldest(min(ST, KT));
+  stage_barrier();
+  frags(lds, 0, 0);
+  for (int kt = 0; kt < KT; ++kt) {
     const TA* sa = lds + (kt % ST) * T::STAGE;
-    V8 af[2][T::TM], wf[2][T::TN];
-    auto frags = [&](int kk, int b) {
-      const int co = ((2 * kk + g) ^ sw) * 8;
-#pragma unroll
-      for (int i = 0; i < T::TM; ++i) af[b][i] = *reinterpret_cast<const V8*>(sa + arow + i * 32 * BK + co);
-#pragma unroll
-      for (int j = 0; j < T::TN; ++j) wf[b][j] = *reinterpret_cast<const V8*>(sa + wrow + j * 32 * BK + co);
-    };
-    frags(0, 0);
 #pragma unroll
     for (int kk = 0; kk < BK / 16; ++kk) {
-      if (kk + 1 < BK / 16) frags(kk + 1, (kk + 1) & 1);
+      if (kk + 1 < BK / 16) {
+        frags(sa, kk + 1, (kk + 1) & 1);
+      } else if (kt + 1 < KT) {
+        wait_oldest(min(ST - 1, KT - 1 - kt));
+        lds_barrier();
+        if (kt + ST < KT) issue(kt % ST, (kt + ST) * BK);
+        frags(lds + ((kt + 1) % ST) * T::STAGE, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < T::TN; ++j)
 #pragma unroll
         for (int i = 0; i < T::TM; ++i) acc[j][i] = mfma32x32x16(wf[kk & 1][j], af[kk & 1][i], acc[j][i]);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
@@ -188,46 +216,68 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dma_kernel(const TA* __restr
   const int wm = wave / WN, wn = wave % WN;
   const int li = lane & 31, g = lane >> 5;
 
-  f32x16 acc[T::TN][T::TM];
-  dma_mainloop<BM, BN, WM, WN, ST>(A, W, M, N, K, m0, n0, smem, acc);
-  __syncthreads();  // every wave is done with the operand stages
-
   // Epilogue in TN slices: slice j holds, for every wave column wn, the 32
   // output columns wn*WTN + j*32 .. +31 (EPW = WN * 32 columns in all), staged
   // as fp32 rows (+ bias), then written 16 bytes per lane (CPL columns: 8 fp16 or 4
   // fp32) with the residual added.  Lane li owns row wm*WTM + i*32 + li and, per
   // register quad q, columns 8q + 4g .. 8q + 4g + 3 of its 32-column block.
+  // What a slice reads from memory (residual, bias) is requested while the slice before
+  // it is written out, the first one's before the k-loop: read pass by pass where it is
+  // used, the fp32 residual of 8192 x 1024 cost a round trip in each of 16 passes.
   float* Cs = reinterpret_cast<float*>(smem);
   constexpr int CPL = 16 / (int)sizeof(TC);  // output columns per lane and store
   constexpr int LPR = T::EPW / CPL;          // lanes per staged row
   constexpr int RPP = NT / LPR;              // rows per pass
+  constexpr int NP = BM / RPP;               // passes
   static_assert(NT % LPR == 0 && BM % RPP == 0 && 32 % CPL == 0, "epilogue geometry");
   const int cl = (tid % LPR) * CPL;                               // column within the slice
   const int ccol = (cl / 32) * T::WTN + (cl % 32);                // column within the tile (+ j*32)
+  struct __attribute__((aligned(CPL * sizeof(TR) < 16 ? CPL * sizeof(TR) : 16))) Chunk {
+    TR e[CPL];
+  };
+  Chunk rv[NP];
+  f32x4 bq[4];
+  auto request = [&](int j) {  // N % 8 == 0: quads and chunks lie wholly inside or outside N
+    if (resid) {
+      const TR* rp = resid + min(n0 + ccol + j * 32, N - CPL);
+#pragma unroll
+      for (int p = 0; p < NP; ++p)
+        rv[p] = *reinterpret_cast<const Chunk*>(rp + min(m0 + tid / LPR + p * RPP, M - 1) * N);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      bq[q] = bias ? *reinterpret_cast<const f32x4*>(bias + min(n0 + wn * T::WTN + j * 32 + 8 * q + 4 * g, N - 4))
+                   : f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  request(0);
+  f32x16 acc[T::TN][T::TM];
+  dma_mainloop<BM, BN, WM, WN, ST>(A, W, M, N, K, m0, n0, smem, acc);
+  __syncthreads();  // every wave is done with the operand stages
+
 #pragma unroll
   for (int j = 0; j < T::TN; ++j) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int scol = wn * 32 + 8 * q + 4 * g;
-      const int tcol = wn * T::WTN + j * 32 + 8 * q + 4 * g;
-      f32x4 bq = {0.f, 0.f, 0.f, 0.f};
-      if (bias) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) bq[e] = n0 + tcol + e < N ? bias[n0 + tcol + e] : 0.f;
-      }
 #pragma unroll
       for (int i = 0; i < T::TM; ++i) {
         const int row = wm * T::WTM + i * 32 + li;
         f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[j][i][4 * q + e] + bq[e];
+        for (int e = 0; e < 4; ++e) v[e] = acc[j][i][4 * q + e] + bq[q][e];
         *reinterpret_cast<f32x4*>(Cs + row * T::LDC + scol) = v;
       }
     }
+    Chunk rc[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) rc[p] = rv[p];
+    if (j + 1 < T::TN) request(j + 1);
     __syncthreads();
     const int n = n0 + ccol + j * 32;
-    if (n < N) {  // N % 8 == 0, so a lane's CPL columns are all in or all out
-      for (int r = tid / LPR; r < BM; r += RPP) {
+    if (n < N) {
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        const int r = tid / LPR + p * RPP;
         const int64_t m = m0 + r;
         if (m >= M) break;
         float v[CPL];
@@ -250,9 +300,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dma_kernel(const TA* __restr
           }
         }
         if (resid) {
-          const TR* rp = resid + m * N + n;
 #pragma unroll
-          for (int e = 0; e < CPL; ++e) v[e] += to_float(rp[e]);
+          for (int e = 0; e < CPL; ++e) v[e] += to_float(rc[p].e[e]);
         }
         if (epi & kEpiMaskResid) {
 #pragma unroll
@@ -283,36 +332,39 @@ static hipError_t launch_dma(const GemmArgs& a) {
   return hipGetLastError();
 }
 
-// Tile choice.  Candidates (measured on MI355X, TFLOP/s at 8192^3 in brackets):
-//   256 x 256, 8 waves of 64 x 128   [1096]  one workgroup per CU
-//   256 x 192, 8 waves of 64 x 96    [ 980]
-//   256 x 128, 8 waves of 64 x 64    [ 951]
-//   128 x 128, 4 waves of 64 x 64    [ 932]  two workgroups per CU
-// Bigger tiles move fewer bytes through LDS and L2 per MFMA, but a grid that
-// ends in a partly filled round wastes CUs.  The estimate below is the number
-// of rounds of tiles times the time of one round (tile area / relative
-// efficiency); it picks 256 x 192 for 8192 x 3072 x 1024 (2 full rounds; +10 %
-// over 128 x 128), 256 x 128 for 8192 x 1024 x 1024 (+6 %) and 256 x 256 for
-// the 3.2 M-row projections (+13-16 %).
+// Tile choice: the candidate with the least estimated time.  n workgroups fall to each CU,
+// per_cu at a time; a group of r takes `fixed` (launch, first loads, epilogue not shared
+// with others) plus per 64-deep k-tile the larger of `step` (one workgroup's chain of LDS
+// reads, products and the barrier) and r x `busy` (its share of the CU's LDS and matrix
+// cores).  The times (us) are fits to MI355X timings of every candidate over M 128 .. 12321,
+// N 216 .. 6144, K 128 .. 2048, where the estimate's choice is at most 11 % slower than the
+// best one.  Small grids are bound by the chain: 1024 x 1024 x 1024 with an fp32 residual
+// takes 31.4 us in 256 x 256 tiles, 15.0 in 128 x 128, 8.5 in 64 x 64 (20.6 with the
+// register-staged kernel that such sizes took before); 2048 x 1024 x 1024 20 -> 11,
+// 300 x 6144 x 2048 30 -> 15.6, 1848 x 216 x 240 10.8 -> 4.5.  Full chips are bound by LDS
+// bandwidth, which big tiles save: 8192 x 1024 x 1024 25 us in 256 x 128, 8192^3 1190
+// TFLOP/s in 256 x 256.
 struct TileCand {
-  int bm, bn, per_cu;  // tile and workgroups resident per CU
-  double eff;          // relative throughput of a full round
+  int bm, bn, per_cu;
+  double fixed, step, busy;
 };
-constexpr TileCand kTiles[] = {{256, 256, 1, 1.00}, {256, 192, 1, 0.90}, {256, 128, 1, 0.87}, {128, 128, 2, 0.85}};
+constexpr TileCand kTiles[] = {{256, 256, 1, 5.5, 1.43, 1.80}, {256, 192, 1, 4.8, 1.09, 1.42},
+                               {256, 128, 1, 4.0, 0.84, 0.98}, {128, 128, 2, 4.0, 0.62, 0.68},
+                               {128, 64, 2, 3.2, 0.43, 0.40},  {64, 128, 2, 3.4, 0.436, 0.39},
+                               {64, 64, 2, 2.8, 0.30, 0.216}};
 
-static int pick_tile(int64_t M, int N) {
+static int pick_tile(int64_t M, int N, int K) {
   const int64_t cus = compute_units();
+  const double kt = (K + 63) / 64;
   int best = 0;
   double best_t = 1e300;
   for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++i) {
     const TileCand& c = kTiles[i];
     const int64_t tiles = ((M + c.bm - 1) / c.bm) * (int64_t)((N + c.bn - 1) / c.bn);
-    const int64_t slots = cus * c.per_cu;
-    const int64_t rounds = (tiles + slots - 1) / slots;
-    // a round with more tiles than CUs shares each CU between per_cu workgroups
-    const double per_round = (double)c.bm * c.bn / c.eff * (tiles > cus ? c.per_cu : 1);
-    const double t = (double)rounds * per_round;
-    if (t < best_t * 0.999) {
+    const int64_t n = (tiles + cus - 1) / cus, rest = n % c.per_cu;
+    auto group = [&](double r) { return c.fixed + kt * (r * c.busy > c.step ? r * c.busy : c.step); };
+    const double t = (double)(n / c.per_cu) * group(c.per_cu) + (rest ? group((double)rest) : 0.0);
+    if (t < best_t) {
       best_t = t;
       best = i;
     }
@@ -322,11 +374,14 @@ static int pick_tile(int64_t M, int N) {
 
 template <typename TR, typename TC, typename TA = f16>
 static hipError_t dispatch_dma(const GemmArgs& a) {
-  switch (pick_tile(a.M, a.N)) {
+  switch (pick_tile(a.M, a.N, a.K)) {
     case 0: return launch_dma<256, 256, 4, 2, 2, 4, TR, TC, TA>(a);
     case 1: return launch_dma<256, 192, 4, 2, 2, 4, TR, TC, TA>(a);
     case 2: return launch_dma<256, 128, 4, 2, 2, 4, TR, TC, TA>(a);
-    default: return launch_dma<128, 128, 2, 2, 2, 8, TR, TC, TA>(a);
+    case 3: return launch_dma<128, 128, 2, 2, 2, 8, TR, TC, TA>(a);
+    case 4: return launch_dma<128, 64, 2, 2, 3, 8, TR, TC, TA>(a);
+    case 5: return launch_dma<64, 128, 2, 2, 3, 8, TR, TC, TA>(a);
+    default: return launch_dma<64, 64, 2, 2, 4, 8, TR, TC, TA>(a);
   }
 }
 
@@ -556,12 +611,10 @@ hipError_t run_gemm_rowln(const GemmRowLnArgs& a) {
 }
 
 bool gemm_dma_ok(const GemmArgs& a) {
-  // K in whole 64-wide k-tiles; N in 8-column groups; a per-block byte offset
-  // (rows x K) that fits 32 bits; at least half a round of 128 x 128 tiles.
-  if (a.ln_gamma || a.K % 64 != 0 || a.N % 8 != 0 || a.M <= 0) return false;
-  if ((int64_t)256 * a.K * 2 >= ((int64_t)1 << 32)) return false;
-  const int64_t tiles = ((a.M + 127) / 128) * (int64_t)((a.N + 127) / 128);
-  return 2 * tiles >= compute_units();
+  // K and N in groups of 8 (16-byte chunks); a per-block byte offset (rows x K) that fits
+  // 32 bits.
+  if (a.ln_gamma || a.K % 8 != 0 || a.N % 8 != 0 || a.M <= 0) return false;
+  return (int64_t)256 * a.K * 2 < ((int64_t)1 << 32);
 }
 
 hipError_t run_gemm_dma(const GemmArgs& a) {

@@ -31,6 +31,10 @@ __device__ __forceinline__ void dma16_untracked(const void* base, uint32_t off, 
                : "s"(lds), "v"(off), "s"(base)
                : "memory");
 }
+// The same from a per-lane address.
+__device__ __forceinline__ void dma16_untracked(const void* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(src) : "memory");
+}
 // LDS byte address of a shared-memory pointer.
 __device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(lds_ptr)p; }
 

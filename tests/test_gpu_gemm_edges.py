@@ -1,0 +1,91 @@
+"""GPU checks of the projection GEMM where tiles, k-tiles and 16-byte chunks end.
+
+Every tile size of the dispatch is reached (small grids take 64 x 64 tiles, larger ones up to
+256 x 256), with M, N and K on both sides of a tile, K down to one 8-element chunk and not a
+multiple of the 64-wide k-tile, residuals and outputs in both widths, bf16, GELU and row
+masks.  Reference: float64 torch on the same 16-bit values.  Tolerances: fp32 outputs
+`sqrt(K) 2^-22` of the largest output (fp32 sums of exact products, in another order); 16-bit
+outputs one unit of roundoff (2^-11, bf16 2^-8) of the value on top.
+"""
+
+import pytest
+import torch
+
+from _gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(M, N, K, dtype=torch.float16, out_fp32=False, resid=None, gelu=False, mask=None):
+    from cobra_amd import ops
+
+    g = torch.Generator().manual_seed(M * 31 + N * 7 + K)
+    a = torch.randn(M, K, generator=g).to(dtype).to(DEV)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(dtype).to(DEV)
+    b = torch.randn(N, generator=g).to(DEV)
+    r = None if resid is None else torch.randn(M, N, generator=g).to(resid).to(DEV)
+    rm = None if mask is None else (torch.rand(M, generator=g) < 0.6).to(DEV)
+    got = ops.linear(a, w, b, gelu=gelu, out_fp32=out_fp32, resid=r, rmask=rm, mask_branch=mask == "branch")
+    want = a.double() @ w.double().t() + b.double()
+    if gelu:
+        want = torch.nn.functional.gelu(want)
+    if mask == "branch":
+        want = want * rm[:, None]
+    if r is not None:
+        want = want + r.double()
+    if mask == "resid":
+        want = want * rm[:, None]
+    unit = 0.0 if out_fp32 else (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8)
+    tol = max(1.0, K ** 0.5) * 2.0 ** -22 * want.abs().max().item() + 2e-6 + unit * want.abs()
+    err = (got.double() - want).abs()
+    assert got.shape == (M, N) and bool((err <= tol).all()), (M, N, K, dtype, (err - tol).max().item())
+
+
+@pytest.mark.parametrize("K", [8, 16, 56, 64, 72, 128, 136, 200, 264, 1032])
+@pytest.mark.parametrize("N", [8, 24, 64, 72, 200, 720])
+def test_small_grids(N, K):
+    for M in (1, 31, 64, 65, 129, 300):
+        _check(M, N, K, out_fp32=True)
+    _check(77, N, K)
+    _check(77, N, K, dtype=torch.bfloat16)
+    _check(130, N, K, out_fp32=True, resid=torch.float32, gelu=True, mask="branch")
+    _check(130, N, K, resid=torch.float16, mask="resid")
+    print(f"[gemm-edges] N{N} K{K} ok", flush=True)
+
+
+@pytest.mark.parametrize("M,N,K", [(2049, 1032, 136), (4100, 1024, 512), (8191, 1024, 72), (8200, 3072, 200),
+                                   (12321, 1536, 512), (16385, 3072, 64), (70000, 136, 128)])
+def test_large_grids(M, N, K):
+    _check(M, N, K)
+    _check(M, N, K, out_fp32=True, resid=torch.float32)
+    _check(M, N, K, dtype=torch.bfloat16, resid=torch.float32)
+    print(f"[gemm-edges] {M}x{N}x{K} ok", flush=True)
+
+
+@pytest.mark.parametrize("K", [8, 72, 200])
+def test_rows_keep_to_themselves(K):
+    """An infinite row of A gives one non-finite output row: the zeros past the end of K are
+    zeros on both operands, not the next row's head."""
+    from cobra_amd import ops
+
+    a = torch.ones(130, K, device=DEV, dtype=torch.float16)
+    a[50] = float("inf")
+    w = torch.ones(72, K, device=DEV, dtype=torch.float16)
+    out = ops.linear(a, w, None, out_fp32=True)
+    finite = torch.isfinite(out).all(1)
+    assert not finite[50] and finite.sum().item() == 129
+    assert bool((out[finite] == K).all())
+
+
+def test_gelu_tail():
+    """GELU far into the negative tail, where 1 + erf cancels: relative to 64 bits."""
+    from cobra_amd import ops
+
+    v = torch.linspace(-5.0, 5.0, 1024, device=DEV).half()
+    a = torch.zeros(1024, 8, device=DEV, dtype=torch.float16)
+    a[:, 0] = v
+    w = torch.zeros(8, 8, device=DEV, dtype=torch.float16)
+    w[:, 0] = 1.0
+    got = ops.linear(a, w, None, gelu=True, out_fp32=True)[:, 3].double()
+    want = v.double() * 0.5 * torch.special.erfc(-v.double() * 0.5 ** 0.5)
+    assert bool(((got - want).abs() <= 4e-6 * want.abs() + 1e-12).all())
