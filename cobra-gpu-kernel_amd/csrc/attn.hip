@@ -525,9 +525,9 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
 // vector pipes: at hd64 each is busy half of the time, and fewer vector instructions, LDS
 // waits or barriers did not move it.
 template <int HD, int NW, int BN, int ST, bool MASKED, typename TQ>
-__global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_causal_kernel(const TQ* __restrict__ qkv, TQ* __restrict__ ctx,
-                                                           int S, int H, int hd, float c2, int nqb,
-                                                           const uint64_t* __restrict__ key_bits, int nwords) {
+__global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_causal_kernel(
+    const TQ* __restrict__ qkv, TQ* __restrict__ ctx, int S, int H, int hd, float c2, int nqb, int nbh,
+    const uint64_t* __restrict__ key_bits, int nwords) {
   using V8 = typename Op16<TQ>::V8;
   using V4 = typename Op16<TQ>::V4;
   using V2 = typename Op16<TQ>::V2;
@@ -560,14 +560,23 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_cau
   __shared__ __attribute__((aligned(1024))) char smem[LDSB];
   char* const qtile = smem + (QSEP ? ST * SB : 0);
 
-  const int id = xcd_remap(blockIdx.x, gridDim.x);
-  // Query block qb visits qb + 1 blocks' worth of keys: of every eight (sequence, head)
-  // pairs the long ones are dispatched first, so that the short ones fill the end.  Eight,
-  // because a group's workgroups share the K / V of its pairs in their XCD's L2.
-  const int grp = id / (8 * nqb), in_grp = id - grp * 8 * nqb;
-  const int pairs = min(8, (int)(gridDim.x / nqb) - 8 * grp);
-  const int qb = nqb - 1 - in_grp / pairs;
-  const int bh = 8 * grp + in_grp % pairs;
+  // Query block qb visits qb + 1 blocks' worth of keys, so every XCD should get an equal
+  // share of each qb, the long ones first, and keep a (sequence, head) pair's K / V in its
+  // L2.  Workgroups go to XCDs round-robin: XCD x takes pairs x, x + 8, .., eight of them at
+  // a time with qb descending (ids past the last pair are empty).  Fewer than 8 pairs: qb
+  // descending over all of them.
+  int qb, bh;
+  if (nbh >= 8) {
+    const int per = (nbh + 7) / 8, l = blockIdx.x / 8;
+    const int grp = l / (8 * nqb), in_grp = l - grp * 8 * nqb;
+    const int pairs = min(8, per - 8 * grp);
+    qb = nqb - 1 - in_grp / pairs;
+    bh = 8 * (8 * grp + in_grp % pairs) + blockIdx.x % 8;
+    if (bh >= nbh) return;
+  } else {
+    qb = nqb - 1 - blockIdx.x / nbh;
+    bh = blockIdx.x % nbh;
+  }
   const int h = bh % H;
   const int64_t b = bh / H;
   const int D = H * hd;
@@ -1067,15 +1076,19 @@ static hipError_t launch_attn_short(const AttnArgs& a, float c2) {
 template <int HD, int NW, int BN, int ST, bool CAUSAL, bool MASKED, typename TQ>
 static hipError_t launch_attn(const AttnArgs& a, float c2) {
   const int nqb = (a.seq_len + 32 * NW - 1) / (32 * NW);
-  const int64_t grid = (int64_t)nqb * a.heads * a.batch;
+  const int64_t nbh = (int64_t)a.heads * a.batch;
+  // The causal kernel deals (sequence, head) pairs to the 8 XCDs: a multiple of 8 of them.
+  const int64_t grid = nqb * (CAUSAL && nbh >= 8 ? (nbh + 7) / 8 * 8 : nbh);
   if (grid > 0x7fffffff) return hipErrorInvalidValue;
-  auto* const kernel = [] {
-    if constexpr (CAUSAL) return attn_causal_kernel<HD, NW, BN, ST, MASKED, TQ>;
-    else return attn_fwd_kernel<HD, NW, BN, ST, MASKED, TQ>;
-  }();
-  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(NW * 64), 0, a.stream, static_cast<const TQ*>(a.qkv),
-                     static_cast<TQ*>(a.ctx), a.seq_len, a.heads, a.head_dim, c2, nqb, a.key_bits,
-                     (int)mask_words(a.seq_len));
+  const TQ* qkv = static_cast<const TQ*>(a.qkv);
+  TQ* ctx = static_cast<TQ*>(a.ctx);
+  const int nwords = (int)mask_words(a.seq_len);
+  if constexpr (CAUSAL)
+    hipLaunchKernelGGL((attn_causal_kernel<HD, NW, BN, ST, MASKED, TQ>), dim3((unsigned)grid), dim3(NW * 64), 0,
+                       a.stream, qkv, ctx, a.seq_len, a.heads, a.head_dim, c2, nqb, (int)nbh, a.key_bits, nwords);
+  else
+    hipLaunchKernelGGL((attn_fwd_kernel<HD, NW, BN, ST, MASKED, TQ>), dim3((unsigned)grid), dim3(NW * 64), 0, a.stream,
+                       qkv, ctx, a.seq_len, a.heads, a.head_dim, c2, nqb, a.key_bits, nwords);
   return hipGetLastError();
 }
 
