@@ -268,6 +268,9 @@ class CobraTransformer(nn.Module):
                                              eps=eps, store_resid=False)[1]
         fused_qkv = ops.qkv_attn_fused(B, S, H, hd)
         r = xf
+        # At these widths the rest of a block is one launch, its fp32 residual updated in place.
+        tail = ops.block_tail_ok(D, cfg.ffn_dim)
+        r_new = torch.empty((T, D), device=x.device, dtype=torch.float32) if tail and n > 1 else None
         for i, p in enumerate(packs):
             last = i == n - 1
             nw, nb = self._final if last else (packs[i + 1].ln1_w, packs[i + 1].ln1_b)
@@ -279,13 +282,19 @@ class CobraTransformer(nn.Module):
             else:
                 qkv = ops.linear(h, p.w_qkv, p.b_qkv)
                 ctx = ops.attn(qkv, B, S, H, hd, scale, causal=cfg.causal, key_bits=bits)
+            norm16 = out16 or not last
+            if tail:
+                r_out = None if last else r_new
+                h = ops.block_tail(ctx, r, p.w_o, p.b_o, p.ln2_w, p.ln2_b, p.w1, p.b1, p.w2, p.b2, nw, nb,
+                                   rmask=mrow, r_out=r_out, norm_fp16=norm16, mask_out=last, eps=eps)
+                r = r_out
+                continue
             if D <= 128:
                 r, h2 = ops.linear_ln(ctx, p.w_o, p.b_o, r, p.ln2_w, p.ln2_b, rmask=mrow, eps=eps, mask_branch=True)
             else:
                 r = ops.linear(ctx, p.w_o, p.b_o, out_fp32=True, resid=r, rmask=mrow, mask_branch=True)
                 _, h2 = ops.add_ln(r, None, None, p.ln2_w, p.ln2_b, cast_fp16=True, eps=eps, store_resid=False)
             hid = ops.linear(h2, p.w1, p.b1, gelu=True)
-            norm16 = out16 or not last
             if D <= 128:
                 r, h = ops.linear_ln(hid, p.w2, p.b2, r, nw, nb, rmask=mrow, norm_fp16=norm16, mask_out=last,
                                      eps=eps)

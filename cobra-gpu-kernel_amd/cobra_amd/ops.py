@@ -295,6 +295,63 @@ def linear_ln(
     return out, normed
 
 
+def block_tail_ok(d_model: int, ffn_dim: int) -> bool:
+    """Whether ``block_tail`` covers a block of these widths."""
+    return d_model == 128 and ffn_dim == 128
+
+
+def block_tail(
+    ctx: torch.Tensor,
+    resid: torch.Tensor,
+    w_o: torch.Tensor,
+    b_o: torch.Tensor,
+    ln2_w: torch.Tensor,
+    ln2_b: torch.Tensor,
+    w1: torch.Tensor,
+    b1: torch.Tensor,
+    w2: torch.Tensor,
+    b2: torch.Tensor,
+    nw: torch.Tensor,
+    nb: torch.Tensor,
+    rmask: Optional[torch.Tensor] = None,
+    r_out: Optional[torch.Tensor] = None,
+    norm_fp16: bool = True,
+    mask_out: bool = False,
+    eps: float = 1e-5,
+) -> torch.Tensor:
+    """A block from its attention's output on, in one launch: ``linear_ln`` (mask_branch)
+    -> ``linear(gelu)`` -> ``linear_ln`` of the reference's loop body (TTB:1255-1290).  Writes
+    the block's fp32 residual to ``r_out`` (may be an fp32 ``resid`` itself; ``None``: not
+    stored, required with ``norm_fp16=False``) and returns the next norm's output.
+    """
+    M, D = ctx.shape
+    F = w1.shape[0]
+    if not block_tail_ok(D, F):
+        raise ValueError(f"block_tail needs d_model = ffn_dim = 128, got {D} and {F}")
+    for name, t, shape in (("ctx", ctx, (M, D)), ("w_o", w_o, (D, D)), ("w1", w1, (F, D)), ("w2", w2, (D, F))):
+        _dev(t, name)
+        if t.dtype != torch.float16 or tuple(t.shape) != shape:
+            raise ValueError(f"{name} must be float16 {list(shape)}")
+    _dev(resid, "resid")
+    if tuple(resid.shape) != (M, D):
+        raise ValueError("resid must have ctx's shape")
+    if r_out is not None:
+        _dev(r_out, "r_out")
+        if r_out.dtype != torch.float32 or tuple(r_out.shape) != (M, D):
+            raise ValueError("r_out must be float32 of ctx's shape")
+    par = [_f32_param(t, D, what) for t, what in (
+        (b_o, "b_o"), (ln2_w, "ln2_w"), (ln2_b, "ln2_b"), (b1, "b1"), (b2, "b2"), (nw, "nw"), (nb, "nb"))]
+    mrow = _row_mask(rmask, M, "rmask")
+    out = torch.empty((M, D), device=ctx.device, dtype=torch.float16 if norm_fp16 else torch.float32)
+    call(
+        "cobra_block_tail_fwd", ctx.data_ptr(), resid.data_ptr(), _dtype_code(resid, "resid"), _ptr(mrow),
+        w_o.data_ptr(), par[0].data_ptr(), par[1].data_ptr(), par[2].data_ptr(), w1.data_ptr(), par[3].data_ptr(),
+        w2.data_ptr(), par[4].data_ptr(), par[5].data_ptr(), par[6].data_ptr(), _ptr(r_out), out.data_ptr(),
+        _dtype_code(out, "out"), 1 if mask_out and mrow is not None else 0, M, D, F, float(eps), _stream(ctx),
+    )
+    return out
+
+
 def ln_linear_ok(d: int, x_dtype: torch.dtype) -> bool:
     """Whether ``ln_linear`` covers rows of width d (one k-tile per row)."""
     return d in (64, 128) and x_dtype in (torch.float16, torch.float32)

@@ -712,4 +712,32 @@ int cobra_block_fwd(const void* h, const float* r, const uint8_t* valid_mask, co
   return code(cobra::run_block_split(a));
 }
 
+int cobra_block_tail_fwd(const void* ctx, const void* resid, int resid_dtype, const uint8_t* row_mask, const void* w_o,
+                         const float* b_o, const float* ln2_w, const float* ln2_b, const void* w1, const float* b1,
+                         const void* w2, const float* b2, const float* lnn_w, const float* lnn_b, float* r_out,
+                         void* out, int out_dtype, int mask_out, int64_t M, int64_t d_model, int64_t ffn_dim,
+                         float eps, void* stream) {
+  if (!cobra::block_tail_ok(d_model, ffn_dim) || M < 0 || !is_dtype(resid_dtype) || !is_dtype(out_dtype)) return kBad;
+  if (M == 0) return 0;
+  const void* must[] = {ctx, resid, w_o, b_o, ln2_w, ln2_b, w1, b1, w2, b2, lnn_w, lnn_b, out};
+  for (const void* p : must)
+    if (!p || !aligned16(p)) return kBad;
+  if (!opt_aligned16(r_out) || (mask_out && !row_mask) || (out_dtype == kF32 && r_out)) return kBad;
+  // A workgroup reads rows ahead of those it writes.
+  auto overlaps = [](const void* x, int64_t nx, const void* y, int64_t ny) {
+    const char *px = static_cast<const char*>(x), *py = static_cast<const char*>(y);
+    return px < py + ny && py < px + nx;
+  };
+  const int64_t hb = M * d_model * 2, rb = M * d_model * dtype_bytes(resid_dtype);
+  const int64_t fb = M * d_model * 4, ob = M * d_model * dtype_bytes(out_dtype);
+  if (overlaps(out, ob, ctx, hb) || overlaps(out, ob, resid, rb)) return kBad;
+  if (r_out && (overlaps(r_out, fb, ctx, hb) || overlaps(r_out, fb, out, ob) ||
+                (!(r_out == resid && resid_dtype == kF32) && overlaps(r_out, fb, resid, rb))))
+    return kBad;
+  cobra::BlockTailArgs a{ctx,  resid, resid_dtype, row_mask, w_o,   w1,    w2,  b_o,       ln2_w,
+                         ln2_b, b1,   b2,          lnn_w,    lnn_b, r_out, out, out_dtype, mask_out ? 1 : 0,
+                         M,    eps,   static_cast<hipStream_t>(stream)};
+  return code(cobra::run_block_tail(a));
+}
+
 }  // extern "C"

@@ -96,10 +96,31 @@ inline int compute_units() {
 }
 
 hipError_t run_gemm(const GemmArgs& a);
-// Plain-epilogue GEMMs through LDS-DMA tiles (K % 64 == 0, N % 8 == 0, at
-// least half a round of 128 x 128 tiles); run_gemm routes eligible shapes there.
+// Plain-epilogue GEMMs through LDS-DMA tiles (K % 8 == 0, N % 8 == 0); run_gemm routes
+// eligible shapes there.
 bool gemm_dma_ok(const GemmArgs& a);
 hipError_t run_gemm_dma(const GemmArgs& a);
+
+// Out-projection, LN2, feed-forward part and the next norm of a transformer block in one
+// launch, d_model = ffn_dim = 128 (block_tail.hip): r1 = resid + mask(ctx W_o^T + b_o);
+// r2 = (r1 + gelu(LN2(r1) W1^T + b1) W2^T + b2) * row_mask -> r_out; out = LNn(r2).
+struct BlockTailArgs {
+  const void* ctx;         // [M, 128] fp16
+  const void* resid;       // [M, 128] resid_dtype (kF16 or kF32); may equal r_out when fp32
+  int resid_dtype;
+  const uint8_t* row_mask; // optional [M]
+  const void *w_o, *w1, *w2;  // [128, 128] fp16
+  const float *b_o, *ln2_w, *ln2_b, *b1, *b2, *lnn_w, *lnn_b;  // [128]
+  float* r_out;            // optional [M, 128]; null when out is fp32
+  void* out;               // [M, 128] out_dtype (kF16 or kF32)
+  int out_dtype;
+  int mask_out;
+  int64_t M;
+  float eps;
+  hipStream_t stream;
+};
+bool block_tail_ok(int64_t d_model, int64_t ffn_dim);
+hipError_t run_block_tail(const BlockTailArgs& a);
 
 // Out-projection with LayerNorm over rows of N = 256 .. 2048 in its epilogue
 // (gemm_dma.hip): y = LN(x + mask(a W^T + bias)) * gamma + beta, a / w / x / y all fp16 or

@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define COBRA_ABI_VERSION 11
+#define COBRA_ABI_VERSION 12
 
 enum { COBRA_F16 = 0, COBRA_F32 = 1, COBRA_BF16 = 2 };
 
@@ -319,6 +319,25 @@ int cobra_block_fwd(const void* h, const float* r, const uint8_t* valid_mask, co
  * torch_transformer_benchmark.py:1030-1071.)
  */
 int cobra_block_plan(int64_t batch, int64_t seq_len, int64_t d_model, int64_t heads, int64_t ffn_dim);
+
+/*
+ * A transformer block from its attention's output on, in one launch (the part of the
+ * reference's _run_fused loop body after the attention, torch_transformer_benchmark.py:
+ * 1255-1290: _tl_linear_ln, _tl_linear(gelu), _tl_linear_ln), for d_model = ffn_dim = 128:
+ *   r1  = resid + mask_branch(ctx W_o^T + b_o)           (fp32)
+ *   f   = gelu(LN2(r1) W1^T + b1)                        (fp16 operands, exact erf GELU)
+ *   r2  = (r1 + f W2^T + b2) * row_valid                 (fp32 -> r_out)
+ *   out = LNn(r2) [* row_valid if mask_out]              (out_dtype)
+ * ctx: [M, 128] fp16; resid: [M, 128] COBRA_F16 or COBRA_F32; row_mask (optional, required
+ * by mask_out): [M] bytes; weights [128, 128] fp16; biases and LayerNorm parameters fp32;
+ * out: COBRA_F16, or COBRA_F32 with r_out NULL.  r_out may be NULL (not stored) or equal an
+ * fp32 resid; otherwise no output may overlap an input.
+ */
+int cobra_block_tail_fwd(const void* ctx, const void* resid, int resid_dtype, const uint8_t* row_mask, const void* w_o,
+                         const float* b_o, const float* ln2_w, const float* ln2_b, const void* w1, const float* b1,
+                         const void* w2, const float* b2, const float* lnn_w, const float* lnn_b, float* r_out,
+                         void* out, int out_dtype, int mask_out, int64_t M, int64_t d_model, int64_t ffn_dim,
+                         float eps, void* stream);
 
 #ifdef __cplusplus
 }
