@@ -719,9 +719,12 @@ int cobra_block_tail_fwd(const void* ctx, const void* resid, int resid_dtype, co
                          float eps, void* stream) {
   if (!cobra::block_tail_ok(d_model, ffn_dim) || M < 0 || !is_dtype(resid_dtype) || !is_dtype(out_dtype)) return kBad;
   if (M == 0) return 0;
-  const void* must[] = {ctx, resid, w_o, b_o, ln2_w, ln2_b, w1, b1, w2, b2, lnn_w, lnn_b, out};
+  const void* must[] = {ctx, resid, w_o, w1, w2, out};
   for (const void* p : must)
     if (!p || !aligned16(p)) return kBad;
+  const float* par[] = {b_o, ln2_w, ln2_b, b1, b2, lnn_w, lnn_b};  // read element by element
+  for (const float* p : par)
+    if (!p || !aligned_to(p, 4)) return kBad;
   if (!opt_aligned16(r_out) || (mask_out && !row_mask) || (out_dtype == kF32 && r_out)) return kBad;
   // A workgroup reads rows ahead of those it writes.
   auto overlaps = [](const void* x, int64_t nx, const void* y, int64_t ny) {

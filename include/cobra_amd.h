@@ -329,7 +329,8 @@ int cobra_block_plan(int64_t batch, int64_t seq_len, int64_t d_model, int64_t he
  *   r2  = (r1 + f W2^T + b2) * row_valid                 (fp32 -> r_out)
  *   out = LNn(r2) [* row_valid if mask_out]              (out_dtype)
  * ctx: [M, 128] fp16; resid: [M, 128] COBRA_F16 or COBRA_F32; row_mask (optional, required
- * by mask_out): [M] bytes; weights [128, 128] fp16; biases and LayerNorm parameters fp32;
+ * by mask_out): [M] bytes; weights [128, 128] fp16; biases and LayerNorm parameters fp32
+ * (4-byte alignment suffices for these, the others are 16-byte aligned);
  * out: COBRA_F16, or COBRA_F32 with r_out NULL.  r_out may be NULL (not stored) or equal an
  * fp32 resid; otherwise no output may overlap an input.
  */

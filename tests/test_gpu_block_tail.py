@@ -115,5 +115,8 @@ def test_arguments():
         _tail(ctx[:, :64].contiguous(), resid, w, par)
     with pytest.raises(ValueError):
         _tail(ctx, resid[:32], w, par)
+    # biases and norm parameters may be views at any element of a larger buffer
+    views = [torch.cat([p.new_zeros(1 + i % 3), p])[1 + i % 3:] for i, p in enumerate(par)]
+    assert torch.equal(_tail(ctx, resid, w, views), _tail(ctx, resid, w, par))
     assert ops.block_tail_ok(128, 128) and not ops.block_tail_ok(128, 512) and not ops.block_tail_ok(256, 128)
     assert _tail(ctx[:0], resid[:0], w, par).shape == (0, D)
