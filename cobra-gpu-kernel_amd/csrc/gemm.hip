@@ -264,6 +264,7 @@ static hipError_t run_gemm_bf16(const GemmArgs& a) {
   const bool rb = !a.resid || a.resid_dtype == kBF16;
   if (!rb && a.resid_dtype != kF32) return hipErrorInvalidValue;
   if (a.c_dtype != kBF16 && a.c_dtype != kF32) return hipErrorInvalidValue;
+  if (gemm_rows128_ok(a)) return run_gemm_rows128(a);
   if (gemm_dma_ok(a)) return run_gemm_dma(a);
   if (a.c_dtype == kBF16) return rb ? dispatch_plain<bf16, bf16, bf16>(a) : dispatch_plain<float, bf16, bf16>(a);
   return rb ? dispatch_plain<bf16, float, bf16>(a) : dispatch_plain<float, float, bf16>(a);
@@ -301,6 +302,7 @@ hipError_t run_gemm(const GemmArgs& a) {
   if (!a.c) return hipErrorInvalidValue;
   const bool c16 = a.c_dtype == kF16;
   if (!c16 && a.c_dtype != kF32) return hipErrorInvalidValue;
+  if (gemm_rows128_ok(a)) return run_gemm_rows128(a);
   if (gemm_dma_ok(a)) return run_gemm_dma(a);
   if (!has_resid || a.resid_dtype == kF16) return c16 ? dispatch_plain<f16, f16>(a) : dispatch_plain<f16, float>(a);
   return c16 ? dispatch_plain<float, f16>(a) : dispatch_plain<float, float>(a);

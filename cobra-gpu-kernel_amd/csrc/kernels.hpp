@@ -173,6 +173,9 @@ hipError_t run_ln_gemm(const LnGemmArgs& a);
 // LayerNorm epilogue for K = 64 / 128 and N = 64 / 128 (ln_gemm.hip); run_gemm
 // routes eligible calls there.
 bool gemm_ln_rows_ok(const GemmArgs& a);
+// Plain projection of 128-wide rows to 384 columns, many rows (ln_gemm.hip, W resident in LDS).
+bool gemm_rows128_ok(const GemmArgs& a);
+hipError_t run_gemm_rows128(const GemmArgs& a);
 hipError_t run_gemm_ln_rows(const GemmArgs& a);
 
 struct AttnArgs {

@@ -397,7 +397,9 @@ hipError_t run_gemm_ln_rows(const GemmArgs& a) {
 // row tiles, so twice the loads and stores are in flight per CU (all of W in LDS
 // leaves room for one workgroup per CU, and the kernel is bound by how many
 // memory operations that workgroup keeps outstanding).
-template <int NT, int BM, int NWV, typename TX, typename TA>
+//
+// NORM false: the rows are operands already (a plain projection, TX = TA).
+template <int NT, int BM, int NWV, typename TX, typename TA, bool NORM = true>
 __global__ __launch_bounds__(64 * NWV) void ln_gemm_p_kernel(const TX* __restrict__ x, const float* __restrict__ gamma,
                                                            const float* __restrict__ beta, const TA* __restrict__ W,
                                                            const float* __restrict__ bias, TA* __restrict__ C,
@@ -443,7 +445,7 @@ __global__ __launch_bounds__(64 * NWV) void ln_gemm_p_kernel(const TX* __restric
     }
   }
   float gv[8], bv[8];
-  load_affine8(gamma, beta, 8 * cl, gv, bv);
+  if constexpr (NORM) load_affine8(gamma, beta, 8 * cl, gv, bv);
   // Bias of this wave's columns in the accumulator layout: tile t, register r ->
   // column 128 t + 32 w + 8 (r / 4) + 4 g + r % 4 (tile t of the four column waves
   // together covers the 128 columns 128 t .. 128 t + 127: q, k, v at N = 384).
@@ -489,22 +491,27 @@ __global__ __launch_bounds__(64 * NWV) void ln_gemm_p_kernel(const TX* __restric
     // ---- LayerNorm of the block's rows into H ----------------------------------------
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) {
-      float xv[8];
-      to_float8(xr[S][p], xv);
-      float s = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) s += xv[e];
-      const float mean = group_sum<CPR>(s) * (1.0f / D);
-      float q = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float t = xv[e] - mean;
-        q += t * t;
-      }
-      const float rstd = rsqrtf(group_sum<CPR>(q) * (1.0f / D) + eps);
       V8 h;
+      if constexpr (NORM) {
+        float xv[8];
+        to_float8(xr[S][p], xv);
+        float s = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) h[e] = (TA)((xv[e] - mean) * rstd * gv[e] + bv[e]);
+        for (int e = 0; e < 8; ++e) s += xv[e];
+        const float mean = group_sum<CPR>(s) * (1.0f / D);
+        float q = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float t = xv[e] - mean;
+          q += t * t;
+        }
+        const float rstd = rsqrtf(group_sum<CPR>(q) * (1.0f / D) + eps);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) h[e] = (TA)((xv[e] - mean) * rstd * gv[e] + bv[e]);
+      } else {
+        static_assert(sizeof(RowChunk<TX>) == sizeof(V8), "rows in the operand type");
+        h = __builtin_bit_cast(V8, xr[S][p]);
+      }
       const int r = RPP * p + rp;
       *reinterpret_cast<V8*>(H + r * ROWB + 16 * (cl ^ (r & 15))) = h;
     }
@@ -594,6 +601,28 @@ static hipError_t launch_ln_gemm_p(const LnGemmArgs& a) {
                        static_cast<const TA*>(a.w), a.bias, static_cast<TA*>(a.c), a.M, a.eps);
   }
   return hipGetLastError();
+}
+
+// A plain projection of 128-wide rows to 384 columns (a QKV projection behind a kernel that
+// has already normalised), no epilogue but the bias, in the operand type.  From two rounds of
+// 64-row blocks on: @@
+bool gemm_rows128_ok(const GemmArgs& a) {
+  return a.K == 128 && a.N == 384 && !a.ln_gamma && !a.resid && a.epi == 0 && a.c && a.c_dtype == a.ab_dtype &&
+         a.M >= (int64_t)64 * 2 * compute_units();
+}
+
+template <typename TA>
+static hipError_t launch_gemm_rows128(const GemmArgs& a) {
+  const int64_t cus = compute_units(), nblk = (a.M + 63) / 64;
+  hipLaunchKernelGGL((ln_gemm_p_kernel<3, 64, 8, TA, TA, false>), dim3((unsigned)(nblk < cus ? nblk : cus)), dim3(512),
+                     0, a.stream, static_cast<const TA*>(a.a), nullptr, nullptr, static_cast<const TA*>(a.w), a.bias,
+                     static_cast<TA*>(a.c), a.M, 0.f);
+  return hipGetLastError();
+}
+
+hipError_t run_gemm_rows128(const GemmArgs& a) {
+  if (!gemm_rows128_ok(a)) return hipErrorInvalidValue;
+  return a.ab_dtype == kBF16 ? launch_gemm_rows128<bf16>(a) : launch_gemm_rows128<f16>(a);
 }
 
 template <int D, typename TX, typename TA>

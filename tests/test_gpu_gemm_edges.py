@@ -62,6 +62,17 @@ def test_large_grids(M, N, K):
     print(f"[gemm-edges] {M}x{N}x{K} ok", flush=True)
 
 
+@pytest.mark.parametrize("M", [32767, 32768, 32769, 32831, 49153, 70001])
+def test_many_rows_of_128_to_384(M):
+    """Both sides of the line where 128 -> 384 columns take the kernel that keeps W in LDS."""
+    _check(M, 384, 128)
+    _check(M, 384, 128, dtype=torch.bfloat16)
+    _check(M, 384, 128, out_fp32=True)
+    _check(M, 384, 128, gelu=True)
+    _check(M, 384, 128, mask="branch")
+    print(f"[gemm-edges] {M}x384x128 ok", flush=True)
+
+
 @pytest.mark.parametrize("K", [8, 72, 200])
 def test_rows_keep_to_themselves(K):
     """An infinite row of A gives one non-finite output row: the zeros past the end of K are
