@@ -101,6 +101,8 @@ __device__ __forceinline__ int swz(int row) {
 
 constexpr float kLazyRescale = 8.0f;    // log2 units
 constexpr float kAcceptSum = 65536.0f;  // a lane's tile sum accepted without a tile maximum
+constexpr float kStartRef = -1.0f;      // log2 units: the causal kernel's reference before a query has one
+constexpr float kStartSum = 32.0f;      // a query's first tile sum accepted against it, one per key of the tile
 
 __device__ __forceinline__ f32x16 splat16(float v) {
   f32x16 r;
@@ -509,7 +511,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
 // The causal form, with or without key masks.  What it does otherwise than the kernel above:
 //   * keys come in pairs of 32-key tiles.  A pair whose keys are all live for every query
 //     of the wave takes the short path: scores, exponentials, products.  The references
-//     start at 0 rather than at a first block's maximum, so a wave's first pair takes it
+//     start at 2^-1 rather than at a first block's maximum, so a wave's first pair takes it
 //     too when its sums lie in fp16's range.  Any other pair goes tile by tile through one
 //     straight line that masks, takes the tile's maximum and rescales; tiles without a live
 //     key are left out, by each wave for itself.
@@ -644,7 +646,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_cau
   // from.  KEEP: repeated in 16 registers as the products' C operand, opaque to the
   // compiler, which would otherwise rebuild the copies for every tile.
   constexpr bool KEEP = PT <= 2 && HD <= 128;
-  f32x16 negm = splat16(0.f);
+  f32x16 negm = splat16(-kStartRef);
   if constexpr (KEEP) asm volatile("" : "+v"(negm));
   float l_run = 0.f;     // this lane's share of the running sum
   bool settled = false;  // every query of the wave has a reference (wave-uniform)
@@ -751,15 +753,19 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_cau
         }
       return lt;
     };
-    // No tile maximum: the probabilities are formed against the query's reference (0 to
-    // begin with) and accepted when every lane's tile sum is at most 2^16, so that no
-    // probability exceeds 2^16 (fp16 holds each one; an fp16 overflow reads as an infinite
-    // sum), and, until every query of the wave has a sum, when each has one of at least
-    // 1/2, so that none is lost at fp16's small end.
+    // No tile maximum: the probabilities are formed against the query's reference and
+    // accepted when every lane's tile sum is at most 2^16, so that no probability exceeds
+    // 2^16 (fp16 holds each one; an fp16 overflow reads as an infinite sum), and, until every
+    // query of the wave has a sum, when each one without a sum gets at least one per key: then
+    // the tile's largest probability is at least 1, as against its own maximum, and no key
+    // comes closer to fp16's small end than it would there.  (The start at 2^-1 is what lets
+    // a tile of ordinary logits, whose sum against 0 is near one per key, pass.)
     auto accepted = [&](float lt, bool first) {
       bool refused = __builtin_amdgcn_ballot_w64(!(lt <= kAcceptSum)) != 0;
-      if (first && !settled)
-        refused = refused || __builtin_amdgcn_ballot_w64(!(sum_xor32(l_run + lt) >= 0.5f)) != 0;
+      if (first && !settled) {
+        const bool enough = sum_xor32(l_run) > 0.f || sum_xor32(lt) >= kStartSum;
+        refused = refused || __builtin_amdgcn_ballot_w64(!enough) != 0;
+      }
       return !refused;
     };
     auto pv = [&](const V8(&pf)[2], uint32_t at) {

@@ -11,6 +11,8 @@ other attention op tests (`allclose(atol=2e-3, rtol=1e-2)`, bf16 `atol=1.6e-2, r
 the rounding of the probabilities and of the output, 2^-11 / 2^-8 of values of order 1).
 """
 
+import math
+
 import pytest
 import torch
 
@@ -84,3 +86,34 @@ def test_masked_attention_repeats_bit_for_bit(hd):
     assert torch.equal(got, ops.attn(x, B, S, H, hd, hd ** -0.5, causal=False, key_mask=mask))
     want = _reference(x, B, S, H, hd, False, mask)
     assert torch.allclose(got.float(), want, atol=8e-3, rtol=1e-2)  # v is twice as large, p up to 1: 4x the rounding
+
+
+@pytest.mark.parametrize("hd", [16, 32, 64, 128])
+@pytest.mark.parametrize("masked", [False, True])
+def test_causal_keys_far_below_a_low_maximum(hd, masked):
+    """A row whose scores all lie below zero: 32 keys near 2^-5.9, thousands near 2^-17.
+
+    Relative to the row's maximum the many are normal fp16 numbers, so each probability is
+    rounded by 2^-11 of itself at most, and the output is off by at most
+    `2^-11 sum_j w_j |v_j - out|` plus its own rounding (2^-11 |out|) and the fp32 sums (2^-18).
+    Relative to 0 they would be subnormal, and the error up to 2^-8 of each."""
+    from cobra_amd import ops
+
+    B, S, H = 1, 4096, 2
+    q, k, v = torch.zeros(3, B, S, H, hd)
+    q[..., 0] = -5.9
+    q[..., 1] = torch.linspace(-17.0, -16.0, S)[None, :, None]
+    k[:, :32, :, 0] = 1.0
+    k[:, 32:, :, 1] = 1.0
+    v[:, 32:] = 1.0
+    x = torch.stack([q, k, v], 2).reshape(B * S, 3 * H * hd).half().to(DEV)
+    mask = (torch.arange(S)[None, :] < S - 3).to(DEV) if masked else None
+    got = ops.attn(x, B, S, H, hd, math.log(2.0), causal=True, key_mask=mask).double()[:, 0]  # log2 units as given
+    few = 32 * 2.0 ** x[:, 0].double()
+    n = (torch.arange(S, device=DEV) - 31).clamp(min=0, max=S - 35 if masked else S)
+    many = n * 2.0 ** x[:, 1].double()
+    few[:31] = 1.0  # rows before the 32nd key: only keys with v = 0
+    out = many / (few + many)
+    tol = 2.0 ** -11 * (2 * out * (1 - out) + out) + 2.0 ** -18
+    err = (got - out).abs()
+    assert bool((err <= tol).all()), (hd, masked, (err / tol).max().item())
