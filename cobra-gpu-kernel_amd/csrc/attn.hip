@@ -756,16 +756,14 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_cau
     // No tile maximum: the probabilities are formed against the query's reference and
     // accepted when every lane's tile sum is at most 2^16, so that no probability exceeds
     // 2^16 (fp16 holds each one; an fp16 overflow reads as an infinite sum), and, until every
-    // query of the wave has a sum, when each one without a sum gets at least one per key: then
-    // the tile's largest probability is at least 1, as against its own maximum, and no key
-    // comes closer to fp16's small end than it would there.  (The start at 2^-1 is what lets
-    // a tile of ordinary logits, whose sum against 0 is near one per key, pass.)
+    // query of the wave has a sum, when each one's comes to one per key of the tile: then the
+    // tile's largest probability is at least 1, as against its own maximum, and no key comes
+    // closer to fp16's small end than it would there.  (The start at 2^-1 is what lets a tile
+    // of ordinary logits, whose sum against 0 is near one per key, pass.)
     auto accepted = [&](float lt, bool first) {
       bool refused = __builtin_amdgcn_ballot_w64(!(lt <= kAcceptSum)) != 0;
-      if (first && !settled) {
-        const bool enough = sum_xor32(l_run) > 0.f || sum_xor32(lt) >= kStartSum;
-        refused = refused || __builtin_amdgcn_ballot_w64(!enough) != 0;
-      }
+      if (first && !settled)
+        refused = refused || __builtin_amdgcn_ballot_w64(!(sum_xor32(l_run + lt) >= kStartSum)) != 0;
       return !refused;
     };
     auto pv = [&](const V8(&pf)[2], uint32_t at) {
