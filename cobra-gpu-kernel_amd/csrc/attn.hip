@@ -111,6 +111,28 @@ __device__ __forceinline__ f32x16 splat16(float v) {
   return r;
 }
 
+// The query block and (sequence, head) pair of a causal workgroup; false: none.  Query block
+// qb visits qb + 1 blocks' worth of keys, so every XCD should get an equal share of each qb,
+// the long ones first, and keep a pair's K / V in its L2.  Workgroups go to XCDs round-robin:
+// XCD x takes an eighth of the pairs, consecutive ones (a sequence's heads share cache lines
+// at head_dim < 64), eight of them at a time with qb descending; ids past its last pair are
+// empty.  Fewer than 8 pairs: qb descending over all of them.
+__device__ __forceinline__ bool deal_causal(int nqb, int nbh, int& qb, int& bh) {
+  if (nbh >= 8) {
+    const int x = blockIdx.x % 8, l = blockIdx.x / 8;
+    const int first = (int)((int64_t)x * nbh / 8), count = (int)((int64_t)(x + 1) * nbh / 8) - first;
+    const int grp = l / (8 * nqb), in_grp = l - grp * 8 * nqb;
+    const int pairs = min(8, count - 8 * grp);
+    if (in_grp >= pairs * nqb) return false;
+    qb = nqb - 1 - in_grp / pairs;
+    bh = first + 8 * grp + in_grp % pairs;
+    return true;
+  }
+  qb = nqb - 1 - blockIdx.x / nbh;
+  bh = blockIdx.x % nbh;
+  return true;
+}
+
 }  // namespace
 
 template <int HD, int NW, int BN, int ST, bool MASKED, typename TQ>
@@ -515,7 +537,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
 //     too when its sums lie in fp16's range.  Any other pair goes tile by tile through one
 //     straight line that masks, takes the tile's maximum and rescales; tiles without a live
 //     key are left out, by each wave for itself.
-//   * query blocks with the most keys are dispatched first (see below).
+//   * query blocks with the most keys are dispatched first (deal_causal).
 //   * the reference is kept as the score products' C operand (16 registers) and LDS
 //     addresses stay in registers; with the masking out of the short path the kernel needs
 //     87-124 registers at head_dim <= 64 where one body with masks needed 124-158, so two
@@ -562,23 +584,8 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_cau
   __shared__ __attribute__((aligned(1024))) char smem[LDSB];
   char* const qtile = smem + (QSEP ? ST * SB : 0);
 
-  // Query block qb visits qb + 1 blocks' worth of keys, so every XCD should get an equal
-  // share of each qb, the long ones first, and keep a (sequence, head) pair's K / V in its
-  // L2.  Workgroups go to XCDs round-robin: XCD x takes pairs x, x + 8, .., eight of them at
-  // a time with qb descending (ids past the last pair are empty).  Fewer than 8 pairs: qb
-  // descending over all of them.
   int qb, bh;
-  if (nbh >= 8) {
-    const int per = (nbh + 7) / 8, l = blockIdx.x / 8;
-    const int grp = l / (8 * nqb), in_grp = l - grp * 8 * nqb;
-    const int pairs = min(8, per - 8 * grp);
-    qb = nqb - 1 - in_grp / pairs;
-    bh = 8 * (8 * grp + in_grp % pairs) + blockIdx.x % 8;
-    if (bh >= nbh) return;
-  } else {
-    qb = nqb - 1 - blockIdx.x / nbh;
-    bh = blockIdx.x % nbh;
-  }
+  if (!deal_causal(nqb, nbh, qb, bh)) return;
   const int h = bh % H;
   const int64_t b = bh / H;
   const int D = H * hd;

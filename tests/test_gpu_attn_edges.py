@@ -117,3 +117,20 @@ def test_causal_keys_far_below_a_low_maximum(hd, masked):
     tol = 2.0 ** -11 * (2 * out * (1 - out) + out) + 2.0 ** -18
     err = (got - out).abs()
     assert bool((err <= tol).all()), (hd, masked, (err / tol).max().item())
+
+
+@pytest.mark.parametrize("B,H", [(1, 7), (2, 4), (3, 3), (13, 5), (11, 7), (100, 3)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_causal_many_pairs(B, H, masked):
+    """Every (sequence, head, query block) is computed: pair counts on both sides of 8 and
+    not in whole groups of 8 per XCD, one to three query blocks."""
+    from cobra_amd import ops
+
+    hd = 32
+    for S in (130, 257, 600):
+        g = torch.Generator().manual_seed(B * 100 + S)
+        x = torch.randn(B * S, 3 * H * hd, generator=g).half().to(DEV)
+        m = _mask("tail", B, S, g).to(DEV) if masked else None
+        got = ops.attn(x, B, S, H, hd, hd ** -0.5, causal=True, key_mask=m).float()
+        want = _reference(x, B, S, H, hd, True, m)
+        assert torch.allclose(got, want, atol=2e-3, rtol=1e-2), (S, (got - want).abs().max().item())
