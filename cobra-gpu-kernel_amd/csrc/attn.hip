@@ -53,6 +53,8 @@
 // q, k, v and ctx are fp16 or bf16 (a template type): the bf16 form uses
 // v_mfma_f32_32x32x16_bf16 and v_dot2_f32_bf16 and rounds the probabilities to
 // bf16, everything else is the same code.
+#include <type_traits>
+
 #include "common.hpp"
 #include "kernels.hpp"
 #include "lds_dma.hpp"
@@ -135,7 +137,8 @@ __device__ __forceinline__ bool deal_causal(int nqb, int nbh, int& qb, int& bh) 
 
 }  // namespace
 
-template <int HD, int NW, int BN, int ST, bool MASKED, typename TQ>
+// IDLE: some wave may lie wholly past S.
+template <int HD, int NW, int BN, int ST, bool IDLE, bool MASKED, typename TQ>
 __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict__ qkv, TQ* __restrict__ ctx,
                                                            int S, int H, int hd, float c2, int nqb,
                                                            const uint64_t* __restrict__ key_bits, int nwords) {
@@ -292,23 +295,9 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
     for (int s = 0; s < ST - 1; ++s)
       if (s < nblk) issue(s, s * BN);
   }
-  for (int n = 0; n < nblk; ++n) {
-    const int kb = n * BN;
-    // Key-validity bits of keys kb .. kb+BN-1 (bit j = key kb + j); the scalar
-    // load completes under the barrier's lgkmcnt wait below.
-    uint64_t kw[KW];
-    if constexpr (MASKED) {
-      const int w0 = kb >> 6;
-      if constexpr (BN == 128) {
-        kw[0] = krow[w0];
-        kw[1] = krow[min(w0 + 1, nwords - 1)];
-        if (w0 + 1 >= nwords) kw[1] = 0;
-      } else if constexpr (BN == 64) {
-        kw[0] = krow[w0];
-      } else {
-        kw[0] = (krow[w0] >> (kb & 32)) & 0xffffffffull;
-      }
-    }
+  // Block n becomes visible to all waves, and block n + ST - 1 is requested into the stage
+  // that every wave is done with.
+  auto advance = [&](int n) {
     // Blocks n+1 .. n+ST-2 may still be in flight; block n must have landed.
     const int ahead = min(ST - 2, nblk - 1 - n);
     if constexpr (ST >= 4) {
@@ -330,7 +319,29 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
     }
     lds_barrier();  // block n visible to all waves; every wave is done with block n-1
     if (n + ST - 1 < nblk) issue((n + ST - 1) % ST, (n + ST - 1) * BN);
-    if (q0w >= S) continue;  // a wave past S only takes part in the transfers and barriers
+  };
+  // A wave past S only takes part in the transfers and barriers, in a loop of its own.
+  const bool idle = IDLE && q0w >= S;
+  if (idle)
+    for (int n = 0; n < nblk; ++n) advance(n);
+  for (int n = idle ? nblk : 0; n < nblk; ++n) {
+    const int kb = n * BN;
+    // Key-validity bits of keys kb .. kb+BN-1 (bit j = key kb + j); the scalar
+    // load completes under the barrier's lgkmcnt wait below.
+    uint64_t kw[KW];
+    if constexpr (MASKED) {
+      const int w0 = kb >> 6;
+      if constexpr (BN == 128) {
+        kw[0] = krow[w0];
+        kw[1] = krow[min(w0 + 1, nwords - 1)];
+        if (w0 + 1 >= nwords) kw[1] = 0;
+      } else if constexpr (BN == 64) {
+        kw[0] = krow[w0];
+      } else {
+        kw[0] = (krow[w0] >> (kb & 32)) & 0xffffffffull;
+      }
+    }
+    advance(n);
     bool kpart = false;      // some key of the block is padded
     if constexpr (MASKED) {
       constexpr uint64_t kFull = BN == 32 ? 0xffffffffull : ~0ull;
@@ -1094,12 +1105,33 @@ static hipError_t launch_attn(const AttnArgs& a, float c2) {
   const TQ* qkv = static_cast<const TQ*>(a.qkv);
   TQ* ctx = static_cast<TQ*>(a.ctx);
   const int nwords = (int)mask_words(a.seq_len);
-  if constexpr (CAUSAL)
+  if constexpr (CAUSAL) {
     hipLaunchKernelGGL((attn_causal_kernel<HD, NW, BN, ST, MASKED, TQ>), dim3((unsigned)grid), dim3(NW * 64), 0,
                        a.stream, qkv, ctx, a.seq_len, a.heads, a.head_dim, c2, nqb, (int)nbh, a.key_bits, nwords);
-  else
-    hipLaunchKernelGGL((attn_fwd_kernel<HD, NW, BN, ST, MASKED, TQ>), dim3((unsigned)grid), dim3(NW * 64), 0, a.stream,
-                       qkv, ctx, a.seq_len, a.heads, a.head_dim, c2, nqb, a.key_bits, nwords);
+  } else {
+    auto launch = [&](auto idle) {
+      hipLaunchKernelGGL((attn_fwd_kernel<HD, NW, BN, ST, decltype(idle)::value, MASKED, TQ>), dim3((unsigned)grid),
+                         dim3(NW * 64), 0, a.stream, qkv, ctx, a.seq_len, a.heads, a.head_dim, c2, nqb, a.key_bits,
+                         nwords);
+    };
+    // Waves past S (IDLE) leave their block only where there are such waves: S1024 and S16384,
+    // which have none, then run as if the loop for them were not there (a test in the one loop
+    // cost 1 %), and B37 S333 hd64 takes 26.2 us, 27.5 with those waves computing.  Masked forms
+    // always have it: the block loop that does not start at a constant keeps 128 registers
+    // where the other one keeps 146 (hd32; 127 and 158 at hd64), and two workgroups share a CU:
+    // B64 S1024 H4 hd32 65.5 -> 52.7 us, B8 S2048 H16 hd64 178 -> 142.  Not at head_dim > 128,
+    // where it loses (B8 S600 hd256 30.9 -> 35.4 us, masked 38.4 -> 42.5), nor with one wave.
+    if constexpr (NW == 1 || HD > 128) {
+      launch(std::false_type{});
+    } else if constexpr (MASKED) {
+      launch(std::true_type{});
+    } else {
+      if (nqb * 32 * NW - a.seq_len >= 32)
+        launch(std::true_type{});
+      else
+        launch(std::false_type{});
+    }
+  }
   return hipGetLastError();
 }
 

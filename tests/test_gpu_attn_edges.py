@@ -72,6 +72,23 @@ def test_attn_edges(hd, causal, kind, offset):
     print(f"[attn-edges] hd{hd} causal={causal} mask={kind} offset={offset} ok", flush=True)
 
 
+@pytest.mark.parametrize("hd", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_noncausal_waves_past_the_end(hd, dt):
+    """Without a mask, on both sides of where a workgroup's last wave has no query, for
+    workgroups of 2, 4 and 8 waves, over one key block and several."""
+    from cobra_amd import ops
+
+    B, H = 3, 2
+    for S in (32, 33, 64, 65, 96, 97, 128, 129, 224, 225, 256, 257, 480, 481, 513, 700):
+        g = torch.Generator().manual_seed(S * 3 + hd)
+        x = torch.randn(B * S, 3 * H * hd, generator=g).to(dt).to(DEV)
+        got = ops.attn(x, B, S, H, hd, hd ** -0.5, causal=False).float()
+        want = _reference(x, B, S, H, hd, False, None)
+        tol = dict(atol=2e-3, rtol=1e-2) if dt == torch.float16 else dict(atol=1.6e-2, rtol=2e-2)
+        assert torch.allclose(got, want, **tol), (hd, S, (got - want).abs().max().item())
+
+
 @pytest.mark.parametrize("hd", [64, 256])
 def test_masked_attention_repeats_bit_for_bit(hd):
     """Sharp logits and a mask ending inside a tile: references move at many places, and two
