@@ -48,8 +48,8 @@
 //   * key masks: the block's validity words are scalar loads (they wait in
 //     lgkmcnt, never behind the K/V transfers in vmcnt).
 //
-// Two kernels share this layout: attn_fwd_kernel for non-causal calls and
-// attn_causal_kernel, where every wave's keys end elsewhere.
+// Two kernels share this layout: attn_fwd_kernel for non-causal calls and all of head_dim
+// over 128, and attn_causal_kernel, where every wave's keys end elsewhere.
 // q, k, v and ctx are fp16 or bf16 (a template type): the bf16 form uses
 // v_mfma_f32_32x32x16_bf16 and v_dot2_f32_bf16 and rounds the probabilities to
 // bf16, everything else is the same code.
@@ -138,9 +138,14 @@ __device__ __forceinline__ bool deal_causal(int nqb, int nbh, int& qb, int& bh) 
 }  // namespace
 
 // IDLE: some wave may lie wholly past S.
-template <int HD, int NW, int BN, int ST, bool IDLE, bool MASKED, typename TQ>
+// CAUSAL: instantiated at head_dim > 128, where attn_causal_kernel's second body takes the
+// registers that O needs: with it (26 to 58 AGPRs beside 256 VGPRs) B8 H8 hd256 took 23.8 us at
+// S300, 35.8 at S512, 76.5 at S1024, 258 at S2048, with this kernel 20.0, 29.1, 61.4 and 202;
+// with key masks 23.4, 38.6, 82.8 and 281 against 23.5, 38.0, 80.4 and 266 (at S130 to S300 up
+// to 0.8 us more).  Query blocks in deal_causal's order: 91 -> 61 us at S1024.
+template <int HD, int NW, int BN, int ST, bool CAUSAL, bool IDLE, bool MASKED, typename TQ>
 __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict__ qkv, TQ* __restrict__ ctx,
-                                                           int S, int H, int hd, float c2, int nqb,
+                                                           int S, int H, int hd, float c2, int nqb, int nbh,
                                                            const uint64_t* __restrict__ key_bits, int nwords) {
   using V8 = typename Op16<TQ>::V8;
   using V4 = typename Op16<TQ>::V4;
@@ -172,9 +177,14 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
   __shared__ __attribute__((aligned(1024))) char smem[LDSB];
   char* const qtile = smem + (QSEP ? ST * SB : 0);
 
-  const int id = xcd_remap(blockIdx.x, gridDim.x);
-  const int qb = id % nqb;
-  const int bh = id / nqb;
+  int qb, bh;
+  if constexpr (CAUSAL) {
+    if (!deal_causal(nqb, nbh, qb, bh)) return;
+  } else {
+    const int id = xcd_remap(blockIdx.x, gridDim.x);
+    qb = id % nqb;
+    bh = id / nqb;
+  }
   const int h = bh % H;
   const int64_t b = bh / H;
   const int D = H * hd;
@@ -188,6 +198,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, li = lane & 31;
   const int q0w = qb * BM + w * 32;  // this wave's first query
+  const int qi = q0w + li;           // this lane's query
 
   // Row-major [rows][HD] tiles in LDS, chunk c of row r at c ^ swz(r), filled by
   // coalesced LDS-DMA: 1 KB span `sp` of a tile holds rows sp*1024/(2HD) ..; each lane
@@ -255,7 +266,8 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
   const int vr = 4 * g + ((lane & 15) >> 2);
   const int vc = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
 
-  const int nblk = (S + BN - 1) / BN;
+  const int kend = CAUSAL ? min(S, (qb + 1) * BM) : S;
+  const int nblk = (kend + BN - 1) / BN;
   const int pre = min(ST - 1, nblk);  // key blocks in flight before the loop
   if constexpr (QSEP) {
 #pragma unroll
@@ -358,8 +370,9 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
     const TQ* Vc = reinterpret_cast<const TQ*>(smem + (n % ST) * SB + TB);
     // s = scores in the exp2 domain minus the running max: the accumulator
     // starts at -m_run (every register of a lane belongs to the lane's query).
-    // Masks only where a block reaches past S or holds a padded key.
-    const bool need_mask = kb + BN > S || kpart;
+    // Masks only where a block reaches past S, causally past this wave's first query, or
+    // holds a padded key.
+    const bool need_mask = kb + BN > S || (CAUSAL && kb + BN > q0w + 1) || kpart;
     auto scores = [&](f32x16(&s)[BN / 32]) {
 #pragma unroll
       for (int t = 0; t < BN / 32; ++t) {
@@ -379,11 +392,11 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
       if constexpr (BN == 32) asm volatile("s_nop 7\n\ts_nop 3" : "+v"(s[0]));
       if (need_mask) {
         // Register r of tile t holds key kb + 4g + kc with kc = 32t + 8(r/4) + r%4,
-        // a constant: the key is past S iff kc > lim.
+        // a constant: the key is past S or causally after the query iff kc > lim.
         // A tile whose keys are all live for every lane of the wave is skipped
         // (a uniform branch per tile, which also keeps the predicates of one tile
         // at a time in scalar registers).
-        const int lim = S - 1 - kb - 4 * g;
+        const int lim = (CAUSAL ? min(S - 1, qi) : S - 1) - kb - 4 * g;
         uint64_t lw[KW];  // this lane's view: bit c = key kb + 32*(word half) + 4g + c
 #pragma unroll
         for (int k = 0; k < KW; ++k) lw[k] = MASKED ? kw[k] >> (4 * g) : 0;
@@ -550,13 +563,13 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
 //     key are left out, by each wave for itself.
 //   * query blocks with the most keys are dispatched first (deal_causal).
 //   * the reference is kept as the score products' C operand (16 registers) and LDS
-//     addresses stay in registers; with the masking out of the short path the kernel needs
-//     87-124 registers at head_dim <= 64 where one body with masks needed 124-158, so two
-//     workgroups of eight waves share a CU.
+//     addresses stay in registers; with the masking out of the short path the eight-wave
+//     forms need 87-124 registers at head_dim <= 64 where one body with masks needed 124-158,
+//     so two of their workgroups share a CU.
 // Measured in one process against that one-body form (us): causal B64 S1024 H4 hd32
 // 60 -> 49, B8 S2048 H16 hd64 140 -> 105, B8 S2048 H8 hd128 141 -> 99, B37 S333 H8 hd64
 // 34 -> 29.  Non-causal calls are no faster in this form (hd32 62 -> 63, hd64 1258 -> 1293 at
-// S16384, hd256 56 -> 69) and keep the kernel above.  Bound by the overlap of the matrix and
+// S16384, hd256 56 -> 69) and keep the kernel above, as does head_dim > 128.  Bound by the overlap of the matrix and
 // vector pipes: at hd64 each is busy half of the time, and fewer vector instructions, LDS
 // waits or barriers did not move it.
 template <int HD, int NW, int BN, int ST, bool MASKED, typename TQ>
@@ -576,11 +589,10 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_cau
   constexpr int NI = SB / 1024;        // 1 KB DMA spans per stage
   constexpr int LPT = NI / NW;         // spans per wave per stage
   constexpr int QPT = BM * HD * 2 / 1024 / NW;  // Q-tile spans per wave
-  static_assert(HD % 16 == 0 && BN % 32 == 0, "tile geometry");
-  static_assert(BN == 32 || BN % 64 == 0, "key-mask words");
-  constexpr int KW = BN > 64 ? BN / 64 : 1;  // validity words per key block
-  constexpr int NTL = BN / 32;         // 32-key tiles per block
-  constexpr int PT = NTL < 2 ? 1 : 2;  // tiles whose scores are in flight together
+  static_assert(HD % 16 == 0 && BN % 64 == 0, "tile geometry, key-mask words");
+  constexpr int KW = BN / 64;   // validity words per key block
+  constexpr int NTL = BN / 32;  // 32-key tiles per block
+  constexpr int PT = 2;         // tiles whose scores are in flight together
   static_assert(NI % (2 * NW) == 0, "every wave DMAs whole spans of each tile");
   // Short-sequence launches (<= 4 waves) give the Q tile its own LDS region, so its
   // DMA overlaps the first K/V stages instead of preceding them; 8-wave launches
@@ -661,11 +673,10 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_cau
 #pragma unroll
   for (int j = 0; j < ND; ++j) o[j] = zero16();
   // The softmax reference of this lane's query, negated: what every score tile starts
-  // from.  KEEP: repeated in 16 registers as the products' C operand, opaque to the
-  // compiler, which would otherwise rebuild the copies for every tile.
-  constexpr bool KEEP = PT <= 2 && HD <= 128;
+  // from, repeated in 16 registers as the products' C operand, opaque to the compiler, which
+  // would otherwise rebuild the copies for every tile.
   f32x16 negm = splat16(-kStartRef);
-  if constexpr (KEEP) asm volatile("" : "+v"(negm));
+  asm volatile("" : "+v"(negm));
   float l_run = 0.f;     // this lane's share of the running sum
   bool settled = false;  // every query of the wave has a reference (wave-uniform)
   const uint64_t* krow = MASKED ? key_bits + b * nwords : nullptr;
@@ -741,7 +752,6 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_cau
         kw[k] = krow[min(wi, nwords - 1)];
         if (wi >= nwords) kw[k] = 0;
       }
-      if constexpr (BN == 32) kw[0] = (kw[0] >> (kb & 32)) | 0xffffffff00000000ull;
     }
     // Blocks n+1 .. n+ST-2 may still be in flight; block n must have landed.
     wait_blocks(min(ST - 2, nblk - 1 - n));
@@ -751,7 +761,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_cau
     const uint32_t base = (n % ST) * SB;
     // Scores of a key tile in the exp2 domain, relative to the queries' references.
     auto scores = [&](f32x16& s, uint32_t at) {
-      s = KEEP ? negm : splat16(negm[0]);
+      s = negm;
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk) s = mfma32x32x16(lds_read16<V8>(ka[kk] + at), qf[kk], s);
     };
@@ -870,13 +880,9 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_cau
           for (int r = 0; r < 16; ++r) o[j][r] *= alpha;
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[r] -= inc;
-        if constexpr (KEEP) {
 #pragma unroll
-          for (int r = 0; r < 16; ++r) negm[r] -= inc;
-          asm volatile("" : "+v"(negm));
-        } else {
-          negm = splat16(negm[0] - inc);
-        }
+        for (int r = 0; r < 16; ++r) negm[r] -= inc;
+        asm volatile("" : "+v"(negm));
         V8 pf[2];
         l_run += probs(s, pf);
         settled = !__builtin_amdgcn_ballot_w64(!(sum_xor32(l_run) > 0.f));
@@ -1099,20 +1105,20 @@ template <int HD, int NW, int BN, int ST, bool CAUSAL, bool MASKED, typename TQ>
 static hipError_t launch_attn(const AttnArgs& a, float c2) {
   const int nqb = (a.seq_len + 32 * NW - 1) / (32 * NW);
   const int64_t nbh = (int64_t)a.heads * a.batch;
-  // The causal kernel deals (sequence, head) pairs to the 8 XCDs: a multiple of 8 of them.
+  // Causal launches deal (sequence, head) pairs to the 8 XCDs: a multiple of 8 of them.
   const int64_t grid = nqb * (CAUSAL && nbh >= 8 ? (nbh + 7) / 8 * 8 : nbh);
   if (grid > 0x7fffffff) return hipErrorInvalidValue;
   const TQ* qkv = static_cast<const TQ*>(a.qkv);
   TQ* ctx = static_cast<TQ*>(a.ctx);
   const int nwords = (int)mask_words(a.seq_len);
-  if constexpr (CAUSAL) {
+  if constexpr (CAUSAL && HD <= 128) {
     hipLaunchKernelGGL((attn_causal_kernel<HD, NW, BN, ST, MASKED, TQ>), dim3((unsigned)grid), dim3(NW * 64), 0,
                        a.stream, qkv, ctx, a.seq_len, a.heads, a.head_dim, c2, nqb, (int)nbh, a.key_bits, nwords);
   } else {
     auto launch = [&](auto idle) {
-      hipLaunchKernelGGL((attn_fwd_kernel<HD, NW, BN, ST, decltype(idle)::value, MASKED, TQ>), dim3((unsigned)grid),
-                         dim3(NW * 64), 0, a.stream, qkv, ctx, a.seq_len, a.heads, a.head_dim, c2, nqb, a.key_bits,
-                         nwords);
+      hipLaunchKernelGGL((attn_fwd_kernel<HD, NW, BN, ST, CAUSAL, decltype(idle)::value, MASKED, TQ>),
+                         dim3((unsigned)grid), dim3(NW * 64), 0, a.stream, qkv, ctx, a.seq_len, a.heads, a.head_dim,
+                         c2, nqb, (int)nbh, a.key_bits, nwords);
     };
     // Waves past S (IDLE) leave their block only where there are such waves: S1024 and S16384,
     // which have none, then run as if the loop for them were not there (a test in the one loop

@@ -151,3 +151,25 @@ def test_causal_many_pairs(B, H, masked):
         got = ops.attn(x, B, S, H, hd, hd ** -0.5, causal=True, key_mask=m).float()
         want = _reference(x, B, S, H, hd, True, m)
         assert torch.allclose(got, want, atol=2e-3, rtol=1e-2), (S, (got - want).abs().max().item())
+
+
+@pytest.mark.parametrize("hd", [136, 256])
+@pytest.mark.parametrize("kind", ["none", "tail", "holes"])
+def test_causal_wide_heads(hd, kind):
+    """head_dim over 128: pair counts on both sides of 8, one to five query blocks of 128, and
+    logits far above the first block's."""
+    from cobra_amd import ops
+
+    for B, H in ((1, 3), (3, 3), (11, 1)):
+        for S in (129, 255, 257, 600):
+            g = torch.Generator().manual_seed(B * 10 + S)
+            q, k, v = torch.randn(3, B, S, H, hd, generator=g)
+            k *= torch.where(torch.arange(S) >= S // 2, 6.0, 1.0)[None, :, None, None]
+            x = torch.stack([q, k, v], 2).reshape(B * S, 3 * H * hd).half().to(DEV)
+            m = _mask(kind, B, S, g)
+            m = None if m is None else m.to(DEV)
+            got = ops.attn(x, B, S, H, hd, hd ** -0.5, causal=True, key_mask=m).float()
+            want = _reference(x, B, S, H, hd, True, m)
+            # probabilities near 1 on values up to 4: 2^-11 of each, and logits of order 20 whose
+            # pre-scaled fp16 queries are off by 2^-11 of them
+            assert torch.allclose(got, want, atol=1.6e-2, rtol=2e-2), (B, S, (got - want).abs().max().item())
