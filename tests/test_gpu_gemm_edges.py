@@ -73,6 +73,20 @@ def test_many_rows_of_128_to_384(M):
     print(f"[gemm-edges] {M}x384x128 ok", flush=True)
 
 
+@pytest.mark.parametrize("N", [1, 7, 9, 65, 130])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_columns_not_in_groups_of_8(N, dtype):
+    """The register-staged kernel, which takes N % 8 != 0: both residual and output widths, GELU,
+    both row masks, K with and without a ragged k-tile, and grids for its 64- and 128-row tiles."""
+    for M, K in ((1, 8), (65, 72), (300, 200), (70001 if N <= 65 else 33000, 64)):
+        for out_fp32 in (False, True):
+            _check(M, N, K, dtype=dtype, out_fp32=out_fp32)
+            _check(M, N, K, dtype=dtype, out_fp32=out_fp32, resid=dtype, gelu=True)
+            _check(M, N, K, dtype=dtype, out_fp32=out_fp32, resid=torch.float32, mask="branch")
+            _check(M, N, K, dtype=dtype, out_fp32=out_fp32, resid=dtype, mask="resid")
+    print(f"[gemm-edges] N{N} {dtype} ok", flush=True)
+
+
 @pytest.mark.parametrize("K", [8, 72, 200])
 def test_rows_keep_to_themselves(K):
     """An infinite row of A gives one non-finite output row: the zeros past the end of K are
