@@ -48,8 +48,8 @@
 //   * key masks: the block's validity words are scalar loads (they wait in
 //     lgkmcnt, never behind the K/V transfers in vmcnt).
 //
-// Two kernels share this layout: attn_fwd_kernel for non-causal calls and all of head_dim
-// over 128, and attn_causal_kernel, where every wave's keys end elsewhere.
+// Two kernels share this layout: attn_fwd_kernel for non-causal calls, all of head_dim over
+// 128 and some short causal ones, and attn_causal_kernel, where every wave's keys end elsewhere.
 // q, k, v and ctx are fp16 or bf16 (a template type): the bf16 form uses
 // v_mfma_f32_32x32x16_bf16 and v_dot2_f32_bf16 and rounds the probabilities to
 // bf16, everything else is the same code.
@@ -118,8 +118,14 @@ __device__ __forceinline__ f32x16 splat16(float v) {
 // the long ones first, and keep a pair's K / V in its L2.  Workgroups go to XCDs round-robin:
 // XCD x takes an eighth of the pairs, consecutive ones (a sequence's heads share cache lines
 // at head_dim < 64), eight of them at a time with qb descending; ids past its last pair are
-// empty.  Fewer than 8 pairs: qb descending over all of them.
+// empty.  Fewer than 8 pairs: qb descending over all of them.  One query block: all alike, and
+// nothing to deal (0.4 us less of 512 x 8 pairs of S64 hd16).
 __device__ __forceinline__ bool deal_causal(int nqb, int nbh, int& qb, int& bh) {
+  if (nqb == 1) {
+    qb = 0;
+    bh = xcd_remap(blockIdx.x, gridDim.x);
+    return true;
+  }
   if (nbh >= 8) {
     const int x = blockIdx.x % 8, l = blockIdx.x / 8;
     const int first = (int)((int64_t)x * nbh / 8), count = (int)((int64_t)(x + 1) * nbh / 8) - first;
@@ -138,8 +144,8 @@ __device__ __forceinline__ bool deal_causal(int nqb, int nbh, int& qb, int& bh) 
 }  // namespace
 
 // IDLE: some wave may lie wholly past S.
-// CAUSAL: instantiated at head_dim > 128, where attn_causal_kernel's second body takes the
-// registers that O needs: with it (26 to 58 AGPRs beside 256 VGPRs) B8 H8 hd256 took 23.8 us at
+// CAUSAL: for some short calls (see dispatch_waves) and head_dim > 128, where attn_causal_kernel's
+// second body takes the registers that O needs: with it (26 to 58 AGPRs beside 256 VGPRs) B8 H8 hd256 took 23.8 us at
 // S300, 35.8 at S512, 76.5 at S1024, 258 at S2048, with this kernel 20.0, 29.1, 61.4 and 202;
 // with key masks 23.4, 38.6, 82.8 and 281 against 23.5, 38.0, 80.4 and 266 (at S130 to S300 up
 // to 0.8 us more).  Query blocks in deal_causal's order: 91 -> 61 us at S1024.
@@ -1101,17 +1107,19 @@ static hipError_t launch_attn_short(const AttnArgs& a, float c2) {
   return hipGetLastError();
 }
 
-template <int HD, int NW, int BN, int ST, bool CAUSAL, bool MASKED, typename TQ>
+// PAIRS: a causal call on attn_causal_kernel.
+template <int HD, int NW, int BN, int ST, bool CAUSAL, bool PAIRS, bool MASKED, typename TQ>
 static hipError_t launch_attn(const AttnArgs& a, float c2) {
   const int nqb = (a.seq_len + 32 * NW - 1) / (32 * NW);
   const int64_t nbh = (int64_t)a.heads * a.batch;
   // Causal launches deal (sequence, head) pairs to the 8 XCDs: a multiple of 8 of them.
-  const int64_t grid = nqb * (CAUSAL && nbh >= 8 ? (nbh + 7) / 8 * 8 : nbh);
+  const int64_t grid = nqb * (CAUSAL && nqb > 1 && nbh >= 8 ? (nbh + 7) / 8 * 8 : nbh);
   if (grid > 0x7fffffff) return hipErrorInvalidValue;
   const TQ* qkv = static_cast<const TQ*>(a.qkv);
   TQ* ctx = static_cast<TQ*>(a.ctx);
   const int nwords = (int)mask_words(a.seq_len);
-  if constexpr (CAUSAL && HD <= 128) {
+  if constexpr (PAIRS) {
+    static_assert(CAUSAL, "causal");
     hipLaunchKernelGGL((attn_causal_kernel<HD, NW, BN, ST, MASKED, TQ>), dim3((unsigned)grid), dim3(NW * 64), 0,
                        a.stream, qkv, ctx, a.seq_len, a.heads, a.head_dim, c2, nqb, (int)nbh, a.key_bits, nwords);
   } else {
@@ -1126,8 +1134,9 @@ static hipError_t launch_attn(const AttnArgs& a, float c2) {
     // always have it: the block loop that does not start at a constant keeps 128 registers
     // where the other one keeps 146 (hd32; 127 and 158 at hd64), and two workgroups share a CU:
     // B64 S1024 H4 hd32 65.5 -> 52.7 us, B8 S2048 H16 hd64 178 -> 142.  Not at head_dim > 128,
-    // where it loses (B8 S600 hd256 30.9 -> 35.4 us, masked 38.4 -> 42.5), nor with one wave.
-    if constexpr (NW == 1 || HD > 128) {
+    // where it loses (B8 S600 hd256 30.9 -> 35.4 us, masked 38.4 -> 42.5), nor with one wave or
+    // causally.
+    if constexpr (NW == 1 || HD > 128 || CAUSAL) {
       launch(std::false_type{});
     } else if constexpr (MASKED) {
       launch(std::true_type{});
@@ -1148,21 +1157,45 @@ static hipError_t launch_attn(const AttnArgs& a, float c2) {
 // 1 KB DMA span per wave per stage (the causal kernel: of the K and of the V tile), and
 // narrow heads take 128-key blocks (half the barriers per key; +7-10 % at head_dim 32,
 // measured).
+//
+// Causal calls take attn_causal_kernel (P) but for
+//   * head_dim > 128;
+//   * four waves (S 65 .. 128) without a mask, where tiles that meet the diagonal are half of the
+//     work and that kernel's one-tile-at-a-time body for them is a longer chain than one body
+//     over the whole block.  More workgroups per CU cover the chain, and from about 7 x 64 /
+//     head_dim of them it is the faster one again: S128 H8 hd64 16.1 against 16.5 us at B128,
+//     25.9 against 25.4 at B256; hd32 15.5 against 16.1 at B256, 26.7 against 26.2 at B512.
+//     At head_dim 65 .. 128 LDS holds one workgroup and it never is (B512 H4 S128 hd96 59.6
+//     against 63.6 us); with a mask it is (S100 hd72 59.9 against 56.7).  At head_dim 16
+//     it is from B128 on (B512 H8 S128 21.3 against 19.2 us) and equal below.
+// Its launches for S <= 128 keep two stages: they have at most two key blocks, and LDS decides how
+// many workgroups share a CU (B2048 H4 hd64: S64 71.6 -> 44.6 us, S32 43.4 -> 32.3, S100 102 ->
+// 88; hd32 27.0 -> 23.4, 18.7 -> 14.7, 50.5 -> 46.1).
 template <int HD, bool CAUSAL, bool MASKED, typename TQ>
 static hipError_t dispatch_waves(const AttnArgs& a, float c2) {
+  constexpr bool P = CAUSAL && HD <= 128;
   constexpr int BN = HD >= 256 ? 32 : 64;
-  constexpr int BN4 = CAUSAL && HD <= 16 ? 128 : BN;
-  constexpr int BN8 = CAUSAL ? (HD <= 16 ? 256 : 128) : (HD <= 32 ? 128 : BN);
-  constexpr int ST = CAUSAL || HD >= 128 ? 3 : 4;
-  constexpr int ST8 = CAUSAL && HD != 32 ? 2 : HD >= 128 ? 3 : 4;
+  constexpr int BN4 = P && HD <= 16 ? 128 : BN;
+  constexpr int BN8 = P ? (HD <= 16 ? 256 : 128) : (HD <= 32 ? 128 : BN);
+  constexpr int STF = HD >= 128 ? 3 : 4;  // attn_fwd_kernel
+  constexpr int ST = P && HD <= 64 ? 2 : STF;
+  constexpr int ST8 = P && HD != 32 ? 2 : STF;
   if constexpr (HD <= 64) {
-    if (a.seq_len <= 32) return launch_attn<HD, 1, BN, ST, CAUSAL, MASKED, TQ>(a, c2);
-    if (a.seq_len <= 64) return launch_attn<HD, 2, BN, ST, CAUSAL, MASKED, TQ>(a, c2);
+    if (a.seq_len <= 32) return launch_attn<HD, 1, BN, ST, CAUSAL, P, MASKED, TQ>(a, c2);
+    if (a.seq_len <= 64) return launch_attn<HD, 2, BN, ST, CAUSAL, P, MASKED, TQ>(a, c2);
   }
   if constexpr (HD <= 128) {
-    if (a.seq_len > 128) return launch_attn<HD, 8, BN8, ST8, CAUSAL, MASKED, TQ>(a, c2);
+    if (a.seq_len > 128) return launch_attn<HD, 8, BN8, ST8, CAUSAL, P, MASKED, TQ>(a, c2);
   }
-  return launch_attn<HD, 4, BN4, ST, CAUSAL, MASKED, TQ>(a, c2);
+  constexpr bool F = P && !MASKED && HD > 16;
+  if constexpr (F && HD > 64) {
+    return launch_attn<HD, 4, BN, STF, CAUSAL, false, MASKED, TQ>(a, c2);
+  } else {
+    if constexpr (F)
+      if ((int64_t)a.batch * a.heads * HD < (int64_t)7 * 64 * compute_units())
+        return launch_attn<HD, 4, BN, STF, CAUSAL, false, MASKED, TQ>(a, c2);
+    return launch_attn<HD, 4, BN4, ST, CAUSAL, P, MASKED, TQ>(a, c2);
+  }
 }
 
 template <int HD, bool CAUSAL, typename TQ>

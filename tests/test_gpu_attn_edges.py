@@ -173,3 +173,27 @@ def test_causal_wide_heads(hd, kind):
             # probabilities near 1 on values up to 4: 2^-11 of each, and logits of order 20 whose
             # pre-scaled fp16 queries are off by 2^-11 of them
             assert torch.allclose(got, want, atol=1.6e-2, rtol=2e-2), (B, S, (got - want).abs().max().item())
+
+
+@pytest.mark.parametrize("hd", [8, 32, 40, 64, 72, 128])
+@pytest.mark.parametrize("pairs", [37, 1800, 3600])
+def test_causal_short(hd, pairs):
+    """Up to 128 tokens, few and many (sequence, head) pairs: both kernels of the dispatch, all
+    workgroup sizes, with and without a mask; logits raised over the sequence, so that later tiles
+    lie above earlier ones."""
+    from cobra_amd import ops
+
+    B, H = (pairs // 4, 4) if pairs > 40 else (pairs, 1)
+    for S in (1, 32, 33, 64, 65, 96, 97, 127, 128):
+        g = torch.Generator(device=DEV).manual_seed(S + pairs)
+        x = torch.randn(B, S, 3, H, hd, generator=g, device=DEV)
+        x[:, S // 2:, 1] *= 3.0
+        x = x.reshape(B * S, 3 * H * hd).half()
+        cpu = torch.Generator().manual_seed(S)
+        for kind in ("none", "tail", "holes"):
+            m = _mask(kind, B, S, cpu)
+            m = None if m is None else m.to(DEV)
+            got = ops.attn(x, B, S, H, hd, hd ** -0.5, causal=True, key_mask=m).float()
+            want = _reference(x, B, S, H, hd, True, m)
+            # probabilities near 1 on values up to 4, logits of order 10 (pre-scaled fp16 queries)
+            assert torch.allclose(got, want, atol=1e-2, rtol=1e-2), (S, kind, (got - want).abs().max().item())
