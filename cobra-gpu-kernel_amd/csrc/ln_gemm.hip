@@ -604,11 +604,13 @@ static hipError_t launch_ln_gemm_p(const LnGemmArgs& a) {
 }
 
 // A plain projection of 128-wide rows to 384 columns (a QKV projection behind a kernel that
-// has already normalised), no epilogue but the bias, in the operand type.  From two rounds of
-// 64-row blocks on: @@
+// has already normalised), no epilogue but the bias, in the operand type.  From 64-row blocks for
+// three quarters of the CUs on; below, the DMA GEMM's smaller tiles reach more of them (replayed
+// in a graph, DMA GEMM against this kernel, us): 4096 rows 4.1 / 5.0, 8192 5.4 / 5.5, 12288 7.4 /
+// 6.0, 16384 7.8 / 6.6, 20480 8.5 / 8.2, 24576 10.5 / 8.5, 32768 11.8 / 9.4, 65536 22.0 / 15.4.
 bool gemm_rows128_ok(const GemmArgs& a) {
   return a.K == 128 && a.N == 384 && !a.ln_gamma && !a.resid && a.epi == 0 && a.c && a.c_dtype == a.ab_dtype &&
-         a.M >= (int64_t)64 * 2 * compute_units();
+         a.M >= (int64_t)64 * 3 * compute_units() / 4;
 }
 
 template <typename TA>

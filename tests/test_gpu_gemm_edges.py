@@ -62,9 +62,10 @@ def test_large_grids(M, N, K):
     print(f"[gemm-edges] {M}x{N}x{K} ok", flush=True)
 
 
-@pytest.mark.parametrize("M", [32767, 32768, 32769, 32831, 49153, 70001])
+@pytest.mark.parametrize("M", [12287, 12288, 12289, 16384, 16385, 32767, 32768, 32769, 32831, 49153, 70001])
 def test_many_rows_of_128_to_384(M):
-    """Both sides of the line where 128 -> 384 columns take the kernel that keeps W in LDS."""
+    """Both sides of the line where 128 -> 384 columns take the kernel that keeps W in LDS, and of
+    whole rounds of its blocks."""
     _check(M, 384, 128)
     _check(M, 384, 128, dtype=torch.bfloat16)
     _check(M, 384, 128, out_fp32=True)
