@@ -115,3 +115,21 @@ def test_gelu_tail():
     got = ops.linear(a, w, None, gelu=True, out_fp32=True)[:, 3].double()
     want = v.double() * 0.5 * torch.special.erfc(-v.double() * 0.5 ** 0.5)
     assert bool(((got - want).abs() <= 4e-6 * want.abs() + 1e-12).all())
+
+
+def test_gelu_far_tail_of_fp32_sums():
+    """GELU of sums with 24 bits, to -9: the exponent v^2 / 2 is rounded twice (2^-24 of it each),
+    and the rest of the formula is good to 2e-6."""
+    from cobra_amd import ops
+
+    v = torch.linspace(-9.0, 9.0, 8192, dtype=torch.float64, device=DEV)
+    hi = v.half()
+    lo = ((v - hi.double()) * 4096.0).half()
+    a = torch.zeros(8192, 8, device=DEV, dtype=torch.float16)
+    a[:, 0], a[:, 1] = hi, lo
+    w = torch.zeros(8, 8, device=DEV, dtype=torch.float16)
+    w[:, 0], w[:, 1] = 1.0, 2.0 ** -12
+    v = (hi.double() + lo.double() * 2.0 ** -12).float().double()  # the sum, rounded once
+    got = ops.linear(a, w, None, gelu=True, out_fp32=True)[:, 3].double()
+    want = v * 0.5 * torch.special.erfc(-v * 0.5 ** 0.5)
+    assert bool(((got - want).abs() <= (v * v * 2.0 ** -24 + 2e-6) * want.abs()).all())
