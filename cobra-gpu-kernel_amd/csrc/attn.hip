@@ -1128,9 +1128,10 @@ static hipError_t launch_attn(const AttnArgs& a, float c2) {
                          dim3((unsigned)grid), dim3(NW * 64), 0, a.stream, qkv, ctx, a.seq_len, a.heads, a.head_dim,
                          c2, nqb, (int)nbh, a.key_bits, nwords);
     };
-    // Waves past S (IDLE) leave their block only where there are such waves: S1024 and S16384,
-    // which have none, then run as if the loop for them were not there (a test in the one loop
-    // cost 1 %), and B37 S333 hd64 takes 26.2 us, 27.5 with those waves computing.  Masked forms
+    // Waves past S (IDLE) leave their block only where they are a sixteenth of all or more:
+    // B37 S333 hd64 takes 26.2 us, 27.5 with those waves computing.  With fewer they compute,
+    // and the loop is as if the one for them were not there (the form that has it costs 0.7 % of
+    // S100000 H16 hd64: 41.06 -> 41.36 ms).  Masked forms
     // always have it: the block loop that does not start at a constant keeps 128 registers
     // where the other one keeps 146 (hd32; 127 and 158 at hd64), and two workgroups share a CU:
     // B64 S1024 H4 hd32 65.5 -> 52.7 us, B8 S2048 H16 hd64 178 -> 142.  Not at head_dim > 128,
@@ -1141,7 +1142,8 @@ static hipError_t launch_attn(const AttnArgs& a, float c2) {
     } else if constexpr (MASKED) {
       launch(std::true_type{});
     } else {
-      if (nqb * 32 * NW - a.seq_len >= 32)
+      const int64_t rows = (int64_t)nqb * 32 * NW, past = rows - a.seq_len;
+      if (past >= 32 && 16 * past >= rows)
         launch(std::true_type{});
       else
         launch(std::false_type{});

@@ -76,11 +76,12 @@ def test_attn_edges(hd, causal, kind, offset):
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 def test_noncausal_waves_past_the_end(hd, dt):
     """Without a mask, on both sides of where a workgroup's last wave has no query, for
-    workgroups of 2, 4 and 8 waves, over one key block and several."""
+    workgroups of 2, 4 and 8 waves, over one key block and several (at 730 the one such wave of
+    24 computes)."""
     from cobra_amd import ops
 
     B, H = 3, 2
-    for S in (32, 33, 64, 65, 96, 97, 128, 129, 224, 225, 256, 257, 480, 481, 513, 700):
+    for S in (32, 33, 64, 65, 96, 97, 128, 129, 224, 225, 256, 257, 480, 481, 513, 700, 730):
         g = torch.Generator().manual_seed(S * 3 + hd)
         x = torch.randn(B * S, 3 * H * hd, generator=g).to(dt).to(DEV)
         got = ops.attn(x, B, S, H, hd, hd ** -0.5, causal=False).float()
