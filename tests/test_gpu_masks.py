@@ -171,7 +171,7 @@ def test_attn_op_key_mask(hd, causal):
 
 @pytest.mark.parametrize("M,N,K", [(8192, 1024, 1024), (300, 96, 40), (4096, 256, 128)])
 def test_linear_epilogue_flags(M, N, K):
-    """GELU, branch mask and residual mask against fp32 torch, on both GEMM kernels."""
+    """GELU, branch mask and residual mask against fp32 torch, on large and small grids."""
     from cobra_amd import ops
 
     torch.manual_seed(M + N)

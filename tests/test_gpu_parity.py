@@ -393,8 +393,7 @@ def test_linear_op():
     (6000, 264, 64, "f16"),         # ragged M and N at the tile-count threshold
 ])
 def test_linear_large_tiles(M, N, K, resid):
-    """Shapes large enough (>= 256 tiles of 256 x 128, K % 64 == 0) for the
-    LDS-DMA GEMM, against an fp32 product."""
+    """Grids large enough for the LDS-DMA GEMM's bigger tiles, against an fp32 product."""
     from cobra_amd import ops
 
     log(f"linear large M{M} N{N} K{K} resid={resid}")
