@@ -158,7 +158,7 @@ __global__ __launch_bounds__(64 * kQaWaves) void qkv_attn_head_kernel(
   // barrier there retires the stage (refilled with tile kt + 2) and the next tile's reads
   // run under those products.  The scheduling barriers keep this order, and untracked DMA the
   // waits for single reads: 66.4 -> 63.1 us at B64 d1024 (non-causal, traced; the layer in a
-  // loop 97.2 -> 94.2 and 95.0 -> 93.1 us on two boxes, equal on two others).  A k-tile now
+  // loop 97.2 -> 94.2 and 95.0 -> 93.1 us on two GPUs, equal on two others).  A k-tile now
   // keeps the matrix cores (1536 cycles), the LDS (168 KB, ~1300) and the load path (56 KB,
   // ~1100) busy for about as long each.
   V8 af[2][2], vf[2], hf[4];
