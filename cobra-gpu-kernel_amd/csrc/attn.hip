@@ -116,24 +116,30 @@ __device__ __forceinline__ f32x16 splat16(float v) {
 // The query block and (sequence, head) pair of a causal workgroup; false: none.  Query block
 // qb visits qb + 1 blocks' worth of keys, so every XCD should get an equal share of each qb,
 // the long ones first, and keep a pair's K / V in its L2.  Workgroups go to XCDs round-robin:
-// XCD x takes an eighth of the pairs, consecutive ones (a sequence's heads share cache lines
-// at head_dim < 64), eight of them at a time with qb descending; ids past its last pair are
-// empty.  Fewer than 8 pairs: qb descending over all of them.  One query block: all alike, and
-// nothing to deal (0.4 us less of 512 x 8 pairs of S64 hd16).
-__device__ __forceinline__ bool deal_causal(int nqb, int nbh, int& qb, int& bh) {
+// an XCD takes an eighth of the pairs, eight of them at a time with qb descending; ids past its
+// last pair are empty.  Which eighth: where a head's rows are whole cache lines, every eighth
+// pair (S179 H16 hd128 B196 172 against 184 us with consecutive ones, S505 H8 hd64 B20 masked 21.1
+// against 21.8), else consecutive pairs, as a sequence's heads share lines (S163 H16 hd96 B58 47.3
+// against 49.6 us, S512 H4 hd32 B64 16.5 against 19.5).  Fewer than 8 pairs: qb descending over all
+// of them.  One query block: all alike, and no ids to spare (0.4 us less of 512 x 8 pairs of S64
+// hd16).
+__device__ __forceinline__ bool deal_causal(int nqb, int nbh, int hd, int& qb, int& bh) {
+  const bool apart = hd % 64 == 0;
   if (nqb == 1) {
     qb = 0;
-    bh = xcd_remap(blockIdx.x, gridDim.x);
+    bh = apart ? (int)blockIdx.x : xcd_remap(blockIdx.x, gridDim.x);
     return true;
   }
   if (nbh >= 8) {
     const int x = blockIdx.x % 8, l = blockIdx.x / 8;
-    const int first = (int)((int64_t)x * nbh / 8), count = (int)((int64_t)(x + 1) * nbh / 8) - first;
+    const int first = (int)((int64_t)x * nbh / 8);
+    const int count = apart ? (nbh + 7 - x) / 8 : (int)((int64_t)(x + 1) * nbh / 8) - first;
     const int grp = l / (8 * nqb), in_grp = l - grp * 8 * nqb;
     const int pairs = min(8, count - 8 * grp);
     if (in_grp >= pairs * nqb) return false;
     qb = nqb - 1 - in_grp / pairs;
-    bh = first + 8 * grp + in_grp % pairs;
+    const int nth = 8 * grp + in_grp % pairs;
+    bh = apart ? 8 * nth + x : first + nth;
     return true;
   }
   qb = nqb - 1 - blockIdx.x / nbh;
@@ -185,7 +191,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const TQ* __restrict_
 
   int qb, bh;
   if constexpr (CAUSAL) {
-    if (!deal_causal(nqb, nbh, qb, bh)) return;
+    if (!deal_causal(nqb, nbh, hd, qb, bh)) return;
   } else {
     const int id = xcd_remap(blockIdx.x, gridDim.x);
     qb = id % nqb;
@@ -614,7 +620,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && HD <= 64 ? 4 : 1) void attn_cau
   char* const qtile = smem + (QSEP ? ST * SB : 0);
 
   int qb, bh;
-  if (!deal_causal(nqb, nbh, qb, bh)) return;
+  if (!deal_causal(nqb, nbh, hd, qb, bh)) return;
   const int h = bh % H;
   const int64_t b = bh / H;
   const int D = H * hd;

@@ -198,3 +198,18 @@ def test_causal_short(hd, pairs):
             want = _reference(x, B, S, H, hd, True, m)
             # probabilities near 1 on values up to 4, logits of order 10 (pre-scaled fp16 queries)
             assert torch.allclose(got, want, atol=1e-2, rtol=1e-2), (S, kind, (got - want).abs().max().item())
+
+
+@pytest.mark.parametrize("hd", [64, 96, 128])
+@pytest.mark.parametrize("B,H", [(1, 7), (3, 3), (13, 5), (100, 3)])
+def test_causal_many_pairs_of_wide_heads(hd, B, H):
+    """The two ways of dealing pairs to the XCDs (heads of whole cache lines, others), one to
+    three query blocks."""
+    from cobra_amd import ops
+
+    for S in (130, 257, 600):
+        g = torch.Generator().manual_seed(B * 100 + S + hd)
+        x = torch.randn(B * S, 3 * H * hd, generator=g).half().to(DEV)
+        got = ops.attn(x, B, S, H, hd, hd ** -0.5, causal=True).float()
+        want = _reference(x, B, S, H, hd, True, None)
+        assert torch.allclose(got, want, atol=2e-3, rtol=1e-2), (S, (got - want).abs().max().item())
