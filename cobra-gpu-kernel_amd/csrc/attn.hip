@@ -1168,6 +1168,12 @@ static hipError_t launch_attn(const AttnArgs& a, float c2) {
 //
 // Causal calls take attn_causal_kernel (P) but for
 //   * head_dim > 128;
+//   * head_dim 17 .. 64 from S512 on, with at most one workgroup per CU (few sequences): nothing
+//     covers a workgroup's own chain then, and the one body's is shorter (B1 H8 hd64 S700 17.0 ->
+//     15.8 us, S3000 56.8 -> 52.5; hd32 S1000 17.2 -> 15.9, S6000 79.8 -> 67.1).  Below S512 the
+//     tiles that this form computes past the diagonal cost more (hd32 S400 9.2 against 10.3).
+//     With a mask only at head_dim <= 32 from S2048 on (S3000 38.8 -> 35.5; S1000 equal, hd64 S3000
+//     49.4 against 50.0); head_dim 128 gains 3 % at most and head_dim 16 loses 3 to 10;
 //   * four waves (S 65 .. 128) without a mask, where tiles that meet the diagonal are half of the
 //     work and that kernel's one-tile-at-a-time body for them is a longer chain than one body
 //     over the whole block.  More workgroups per CU cover the chain, and from about 7 x 64 /
@@ -1191,6 +1197,11 @@ static hipError_t dispatch_waves(const AttnArgs& a, float c2) {
   if constexpr (HD <= 64) {
     if (a.seq_len <= 32) return launch_attn<HD, 1, BN, ST, CAUSAL, P, MASKED, TQ>(a, c2);
     if (a.seq_len <= 64) return launch_attn<HD, 2, BN, ST, CAUSAL, P, MASKED, TQ>(a, c2);
+  }
+  if constexpr (P && HD > 16 && HD <= (MASKED ? 32 : 64)) {
+    const int64_t grid = (int64_t)((a.seq_len + 255) / 256) * a.batch * a.heads;
+    if (a.seq_len >= (MASKED ? 2048 : 512) && grid <= compute_units())
+      return launch_attn<HD, 8, HD <= 32 ? 128 : BN, STF, CAUSAL, false, MASKED, TQ>(a, c2);
   }
   if constexpr (HD <= 128) {
     if (a.seq_len > 128) return launch_attn<HD, 8, BN8, ST8, CAUSAL, P, MASKED, TQ>(a, c2);
