@@ -22,7 +22,7 @@ Also on the same line:
     shapes with bf16 activations (the staged kernels with bf16 operands);
   * ``model``: the whole ``CobraTransformer`` stack on three of the reference's
     model cases (tools/sweep.py:31-47), causal, fp16;
-  * ``measured_peaks``: fp16 GEMM TFLOP/s and device-copy GB/s on this box;
+  * ``measured_peaks``: fp16 GEMM TFLOP/s and device-copy GB/s on this machine;
   * ``graph``: the same forward replayed as a hipGraph, and an empty-graph floor.
 
 Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-long] [--no-cpu] [--no-sweep]
@@ -156,7 +156,7 @@ def roofline(name, flops, nbytes, ms, peak_tflops=PEAK_FP16_TFLOPS, peak_gbs=PEA
 
 
 def measured_peaks(dev):
-    """Sustained fp16 GEMM and copy rates of this box, for the "% of measured peak" figures.
+    """Sustained fp16 GEMM and copy rates of this machine, for the "% of measured peak" figures.
 
     The GEMM is 8192^3 through torch (hipBLASLt) in the layout every projection
     on the path uses (A [M, K] row-major times W^T, W [N, K] row-major), on
@@ -207,7 +207,7 @@ def cpu_model() -> str:
 
 def host_info() -> dict:
     """The host CPU the baselines ran on.  `cores` on the baselines is the thread count
-    torch used (the box's CPU share: OMP_NUM_THREADS), not the machine's core count."""
+    torch used (the CPU share: OMP_NUM_THREADS), not the machine's core count."""
     return {"cpu_model": cpu_model(), "os_cpu_count": os.cpu_count(), "torch_threads": torch.get_num_threads()}
 
 
